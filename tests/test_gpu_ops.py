@@ -259,6 +259,28 @@ def test_matmul_dispatch(ctx, orc):
         assert_bits(ctx.download(od, np.float32, rows), want)
 
 
+# Q8_0: fewer rows than a work group's 8, one row past it; one block, a last step of one block, whole
+# 256-block chunks, one block past them.  F32: fewer columns than a wave, one short of and past a 16-load
+# batch, a ragged tail.  x starts at 4-byte offsets: neither kernel may need more.
+@pytest.mark.parametrize("gtype,rows,cols,off", [
+    (mcpm.TYPE_Q8_0, 1, 32, 0), (mcpm.TYPE_Q8_0, 7, 33 * 32, 1), (mcpm.TYPE_Q8_0, 9, 256 * 32, 3),
+    (mcpm.TYPE_Q8_0, 17, 257 * 32, 2), (mcpm.TYPE_Q8_0, 2304, 5760, 0),
+    (mcpm.TYPE_F32, 1, 1, 1), (mcpm.TYPE_F32, 5, 63, 2), (mcpm.TYPE_F32, 6, 1023, 3), (mcpm.TYPE_F32, 3, 1025, 1),
+    (mcpm.TYPE_F32, 70, 2111, 0)])
+def test_gemv_f32_activations_bit_exact(ctx, orc, gtype, rows, cols, off):
+    rng = np.random.default_rng(rows * 31 + cols)
+    blk = rand_q8_0(rng, rows * cols // 32) if gtype == mcpm.TYPE_Q8_0 else rng.standard_normal((rows, cols)).astype(np.float32).ravel()
+    x = rand_act(rng, cols)
+    announce(f"f32-activation gemv type={gtype} {rows}x{cols} x+{4 * off}")
+    t = ctx.tensor(blk, gtype, cols, rows)
+    xd = up(ctx, np.concatenate([np.zeros(off, np.float32), x]))
+    od = ctx.zeros(rows * 4)
+    mcpm.check(ctx.lib.mcpm_matmul(ctx.h, t.h, xd.ptr + 4 * off, od.ptr))
+    want = np.zeros(rows, np.float32)
+    assert orc.or_matmul(gtype, P(blk), P(x), P(want), rows, cols) == 0
+    assert_bits(ctx.download(od, np.float32, rows), want)
+
+
 def test_unsupported_type_rejected(ctx):
     with pytest.raises(mcpm.McpmError) as ei:
         ctx.tensor(np.zeros(256 * 2, np.uint8), 1, 256, 1)  # F16
