@@ -23,82 +23,125 @@ namespace mcpm {
 
 // ------------------------------------------------------- standalone ops ----
 
-// Q8_K blocks of an fp32 vector (optionally RMS-normalised) in native layout.
-// mode: PRO_QUANT_EVEN / PRO_QUANT_AWAY / PRO_NORM_AWAY / PRO_NORM_EVEN.
-__global__ void __launch_bounds__(256) k_quantize_q8k(const float* __restrict__ x, const float* __restrict__ gamma,
-                                                      float eps, int dim, int mode, BlockQ8K* __restrict__ out) {
-  __shared__ float red[260];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const bool norm = (mode == PRO_NORM_AWAY || mode == PRO_NORM_EVEN);
-  const bool away = (mode == PRO_QUANT_AWAY || mode == PRO_NORM_AWAY);
-  float rms = 1.0f;
-  if (norm) rms = block_rms_scale(x, dim, eps, red);
-  const int nb = dim / QK_K;
-  for (int b = wave; b < nb; b += 4) {
-    const float4 xv = reinterpret_cast<const float4*>(x + b * QK_K)[lane];
-    float v[4] = {xv.x, xv.y, xv.z, xv.w};
-    if (norm) {
-      const float4 gv = reinterpret_cast<const float4*>(gamma + b * QK_K)[lane];
-      v[0] = (v[0] * rms) * gv.x;
-      v[1] = (v[1] * rms) * gv.y;
-      v[2] = (v[2] * rms) * gv.z;
-      v[3] = (v[3] * rms) * gv.w;
-    }
-    uint32_t packed;
-    float d;
-    int gsum;
-    quant_block_wave(v, away, packed, d, gsum);
-    reinterpret_cast<uint32_t*>(out[b].qs)[lane] = packed;
-    if ((lane & 3) == 0) out[b].bsums[lane >> 2] = static_cast<int16_t>(gsum);
-    if (lane == 0) out[b].d = d;
+// One wave's 256-value block (lane l: values 4l .. 4l+3) quantized into out.
+__device__ __forceinline__ void store_q8k_block(const float (&v)[4], bool away, int lane, BlockQ8K* __restrict__ out) {
+  uint32_t packed;
+  float d;
+  int gsum;
+  quant_block_wave(v, away, packed, d, gsum);
+  reinterpret_cast<uint32_t*>(out->qs)[lane] = packed;
+  if ((lane & 3) == 0) out->bsums[lane >> 2] = static_cast<int16_t>(gsum);
+  if (lane == 0) out->d = d;
+}
+
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // float vectors have no alignment of their own
+
+// Q8_K blocks of an fp32 vector in native layout, one wave (work group) per block.
+__global__ void __launch_bounds__(64) k_quantize_q8k(const float* __restrict__ x, bool away,
+                                                     BlockQ8K* __restrict__ out) {
+  const int b = blockIdx.x, lane = threadIdx.x;
+  const f32x4_u xv = *reinterpret_cast<const f32x4_u*>(x + b * QK_K + 4 * lane);
+  const float v[4] = {xv.x, xv.y, xv.z, xv.w};
+  store_q8k_block(v, away, lane, out + b);
+}
+
+// Q8_K blocks of the RMS-normalised vector, a work group per block: each reads
+// the whole vector (its gammas with it, so there is one trip to memory) and
+// forms the sum of squares itself, then its first wave quantizes the work
+// group's block.  NV: values per thread, dim <= 256 * NV.  One work group for
+// all blocks ran them three deep after two more trips to memory: 4.8 -> 3.1 us
+// at 2048 and 2304 values.
+template <int NV>
+__global__ void __launch_bounds__(256) k_norm_quantize_q8k(const float* __restrict__ x,
+                                                           const float* __restrict__ gamma, float eps, int dim,
+                                                           bool away, BlockQ8K* __restrict__ out) {
+  __shared__ float red[256];
+  const int tid = threadIdx.x, b = blockIdx.x;
+  f32x4_u xb = {}, gb = {};
+  if (tid < 64) {
+    xb = *reinterpret_cast<const f32x4_u*>(x + b * QK_K + 4 * tid);
+    gb = *reinterpret_cast<const f32x4_u*>(gamma + b * QK_K + 4 * tid);
+  }
+  float p = 0.0f;
+  for (int i0 = 0; i0 < dim; i0 += 256 * NV) {
+    float v[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = x[min(i0 + tid + 256 * k, dim - 1)];
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (i0 + tid + 256 * k < dim) p = p + v[k] * v[k];
+  }
+  const float rms = block_rms_1sync(p, dim, eps, red);
+  if (tid < 64) {
+    const float v[4] = {(xb.x * rms) * gb.x, (xb.y * rms) * gb.y, (xb.z * rms) * gb.z, (xb.w * rms) * gb.w};
+    store_q8k_block(v, away, tid, out + b);
   }
 }
 
 hipError_t launch_quantize_q8k(const float* x, const float* gamma, float eps, int dim, int mode, BlockQ8K* out,
                                hipStream_t s) {
-  hipLaunchKernelGGL(k_quantize_q8k, dim3(1), dim3(256), 0, s, x, gamma, eps, dim, mode, out);
+  const bool norm = (mode == PRO_NORM_AWAY || mode == PRO_NORM_EVEN);
+  const bool away = (mode == PRO_QUANT_AWAY || mode == PRO_NORM_AWAY);
+  const dim3 grid(dim / QK_K);
+  if (!norm)
+    hipLaunchKernelGGL(k_quantize_q8k, grid, dim3(64), 0, s, x, away, out);
+  else
+    hipLaunchKernelGGL(k_norm_quantize_q8k<12>, grid, dim3(256), 0, s, x, gamma, eps, dim, away, out);
   return hipGetLastError();
 }
 
-// rmsnorm (src/ops/ops.cpp:468-481): out = (x*rms)*w.
-__global__ void __launch_bounds__(256) k_rmsnorm(const float* __restrict__ x, const float* __restrict__ w, float eps,
-                                                 int dim, float* __restrict__ out) {
-  __shared__ float red[260];
-  const float rms = block_rms_scale(x, dim, eps, red);
-  for (int i = threadIdx.x; i < dim; i += 256) out[i] = (x[i] * rms) * w[i];
+// rmsnorm (src/ops/ops.cpp:468-481): out = (x*rms)*w.  One work group, which
+// reads all of x before it writes (out may be x).  Up to NV values a thread
+// stay in registers with their weights, so the vector is read once; the
+// second trip to memory is for longer ones only (2304 values: 4.1 -> 3.1 us).
+template <int NV>
+__global__ void __launch_bounds__(256) k_rmsnorm(const float* x, const float* __restrict__ w, float eps, int dim,
+                                                 float* out) {
+  __shared__ float red[256];
+  const int tid = threadIdx.x;
+  float v[NV], g[NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    v[k] = x[min(tid + 256 * k, dim - 1)];
+    g[k] = w[min(tid + 256 * k, dim - 1)];
+  }
+  float p = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if (tid + 256 * k < dim) p = p + v[k] * v[k];
+  for (int i = tid + 256 * NV; i < dim; i += 256) p = p + x[i] * x[i];
+  const float rms = block_rms_1sync(p, dim, eps, red);
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if (tid + 256 * k < dim) out[tid + 256 * k] = (v[k] * rms) * g[k];
+  for (int i = tid + 256 * NV; i < dim; i += 256) out[i] = (x[i] * rms) * w[i];
 }
 
 hipError_t launch_rmsnorm(const float* x, const float* w, float eps, int dim, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_rmsnorm, dim3(1), dim3(256), 0, s, x, w, eps, dim, out);
+  hipLaunchKernelGGL(k_rmsnorm<12>, dim3(1), dim3(256), 0, s, x, w, eps, dim, out);
   return hipGetLastError();
 }
 
-// swiglu_and_quantize_q8k (src/ops/ops.cpp:725-765): dim/256 blocks, lround.
-__global__ void __launch_bounds__(256) k_swiglu_quant(const float* __restrict__ g, const float* __restrict__ u, int dim,
-                                                      BlockQ8K* __restrict__ out) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int nb = dim / QK_K;
-  for (int b = wave; b < nb; b += 4) {
-    float v[4];
+// swiglu_and_quantize_q8k (src/ops/ops.cpp:725-765): dim/256 blocks, lround,
+// one wave (work group) per block.  One work group for all blocks took them
+// six deep, with four scalar loads of each vector: 10.0 -> 2.6 us at 5888 values.
+__global__ void __launch_bounds__(64) k_swiglu_quant(const float* __restrict__ g, const float* __restrict__ u,
+                                                     BlockQ8K* __restrict__ out) {
+  const int b = blockIdx.x, lane = threadIdx.x;
+  const f32x4_u gv = *reinterpret_cast<const f32x4_u*>(g + b * QK_K + 4 * lane);
+  const f32x4_u uv = *reinterpret_cast<const f32x4_u*>(u + b * QK_K + 4 * lane);
+  float v[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int i = b * QK_K + 4 * lane + k;
-      const float gg = g[i];
-      const float silu = gg / (1.0f + exp_f32(-gg));
-      v[k] = silu * u[i];
-    }
-    uint32_t packed;
-    float d;
-    int gsum;
-    quant_block_wave(v, true, packed, d, gsum);
-    reinterpret_cast<uint32_t*>(out[b].qs)[lane] = packed;
-    if ((lane & 3) == 0) out[b].bsums[lane >> 2] = static_cast<int16_t>(gsum);
-    if (lane == 0) out[b].d = d;
+  for (int k = 0; k < 4; ++k) {
+    const float gg = gv[k];
+    const float silu = gg / (1.0f + exp_f32(-gg));
+    v[k] = silu * uv[k];
   }
+  store_q8k_block(v, true, lane, out + b);
 }
 
 hipError_t launch_swiglu_quant(const float* g, const float* u, int dim, BlockQ8K* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_swiglu_quant, dim3(1), dim3(256), 0, s, g, u, dim, out);
+  hipLaunchKernelGGL(k_swiglu_quant, dim3(dim / QK_K), dim3(64), 0, s, g, u, out);
   return hipGetLastError();
 }
 
@@ -555,25 +598,50 @@ __global__ void __launch_bounds__(256) k_attention_tile(const float* __restrict_
 
 // The combine over a head's chunks for output i (head h, dim d), in chunk
 // order: m = max m_c; f_c = exp(m_c - m); Z = fma(z_c, f_c, Z);
-// O = fma(o_c[d], f_c, O); out = O / Z.
-__global__ void k_attn_combine(const float* __restrict__ part_o, const float2* __restrict__ part_mz,
-                               const int* __restrict__ state, int n_out, int hd, int max_chunks,
-                               float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_out) return;
+// O = fma(o_c[d], f_c, O); out = O / Z.  One wave per 64 outputs of a head.
+// Lane c holds chunk c's (m_c, z_c) and forms f_c once for the wave (each
+// output formed every f_c itself before, an exp between each two loads); the
+// chains read it by lane, and the o_c of COMBINE_BATCH chunks are loaded
+// together.  Average over 32 heads of 64 at 9 chunks and 16 of 128 at 63: 22.9 ->
+// 4.5 us.
+constexpr int COMBINE_BATCH = 16;
+
+__global__ void __launch_bounds__(64) k_attn_combine(const float* __restrict__ part_o,
+                                                     const float2* __restrict__ part_mz,
+                                                     const int* __restrict__ state, int hd, int max_chunks,
+                                                     float* __restrict__ out) {
   const int nch = state[1] / ATTN_CHUNK + 1;
-  const int h = i / hd, d = i - h * hd;
+  const int h = blockIdx.x, lane = threadIdx.x, d = blockIdx.y * 64 + lane;
   const float2* mz = part_mz + static_cast<size_t>(h) * max_chunks;
-  const float* o = part_o + static_cast<size_t>(h) * max_chunks * hd + d;
-  float m = mz[0].x;
-  for (int c = 1; c < nch; ++c) m = fmaxf(m, mz[c].x);
+  // lanes past the head's dims repeat its last one (unused)
+  const float* o = part_o + static_cast<size_t>(h) * max_chunks * hd + min(d, hd - 1);
+  // lanes past the last chunk hold it again: the maximum is unchanged, and
+  // the chains stop before them
+  float2 cur = mz[min(lane, nch - 1)];
+  float m = cur.x;
+  for (int c0 = 64; c0 < nch; c0 += 64) m = fmaxf(m, mz[min(c0 + lane, nch - 1)].x);
+  m = wave_max_fast(m);
   float Z = 0.0f, O = 0.0f;
-  for (int c = 0; c < nch; ++c) {
-    const float f = exp_f32(mz[c].x - m);
-    Z = __builtin_fmaf(mz[c].y, f, Z);
-    O = __builtin_fmaf(o[static_cast<size_t>(c) * hd], f, O);
+  for (int c0 = 0; c0 < nch; c0 += 64) {
+    if (c0 > 0) cur = mz[min(c0 + lane, nch - 1)];
+    const float f = exp_f32(cur.x - m);
+    const int n = min(64, nch - c0);
+    for (int j0 = 0; j0 < n; j0 += COMBINE_BATCH) {
+      float ov[COMBINE_BATCH];
+#pragma unroll
+      for (int k = 0; k < COMBINE_BATCH; ++k) ov[k] = o[static_cast<size_t>(min(c0 + j0 + k, nch - 1)) * hd];
+#pragma unroll
+      for (int k = 0; k < COMBINE_BATCH; ++k) {
+        if (j0 + k < n) {  // uniform
+          const float fc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), j0 + k));
+          const float zc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cur.y), j0 + k));
+          Z = __builtin_fmaf(zc, fc, Z);
+          O = __builtin_fmaf(ov[k], fc, O);
+        }
+      }
+    }
   }
-  out[i] = O / Z;
+  if (d < hd) out[static_cast<size_t>(h) * hd + d] = O / Z;
 }
 
 hipError_t launch_attention(const float* q, const float* kc, const float* vc, const int* state, int n_heads,
@@ -634,9 +702,8 @@ hipError_t launch_attention_batch(const float* q, const float* kc, const float* 
 
 hipError_t launch_attn_combine(const AttnPart& part, const int* state, int n_heads, int head_dim, int max_chunks,
                                float* out, hipStream_t s) {
-  const int n = n_heads * head_dim;
-  hipLaunchKernelGGL(k_attn_combine, dim3((n + 255) / 256), dim3(256), 0, s, part.o, part.mz, state, n, head_dim,
-                     max_chunks, out);
+  hipLaunchKernelGGL(k_attn_combine, dim3(n_heads, (head_dim + 63) / 64), dim3(64), 0, s, part.o, part.mz, state,
+                     head_dim, max_chunks, out);
   return hipGetLastError();
 }
 
@@ -754,8 +821,6 @@ hipError_t launch_stream_read(const void* src, size_t bytes, int grid, uint32_t*
 // rate).  One lane per whole row gave 9 work groups at 2304 rows: 2304 x 5760 52.7 -> 7.6 us,
 // 1000 x 1024 10.8 -> 3.8, 8192 x 6144 87.0 -> 20.9 (53.7 MB, 2.6 TB/s).
 constexpr int Q80_ROWS = 8, Q80_PAR = 256 / Q80_ROWS, Q80_CHUNK = 256;
-
-typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // x has no alignment of its own
 
 __global__ void __launch_bounds__(256) k_gemv_q8_0(const WView w, const float* __restrict__ x,
                                                    float* __restrict__ out, int rows, int cols) {

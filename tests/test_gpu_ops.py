@@ -133,6 +133,19 @@ def test_rmsnorm_ops(ctx, orc, dim):
     assert_bits(ctx.download(qd, mcpm.Q8_K, dim // 256), wq)
 
 
+# fewer values than threads, one past the 3072 a work group keeps in registers, a ragged tail; out is x
+@pytest.mark.parametrize("dim", [1, 255, 3073, 6000])
+def test_rmsnorm_in_place(ctx, orc, dim):
+    rng = np.random.default_rng(dim)
+    x, w = rand_act(rng, dim, 2.0), rand_act(rng, dim, 1.0)
+    announce(f"rmsnorm in place dim={dim}")
+    xd = up(ctx, np.concatenate([np.zeros(1, np.float32), x]))  # a 4-byte offset
+    mcpm.check(ctx.lib.mcpm_rmsnorm(ctx.h, xd.ptr + 4, xd.ptr + 4, up(ctx, w).ptr, dim, 1e-6))
+    want = np.zeros(dim, np.float32)
+    orc.or_rmsnorm(P(want), P(x), P(w), dim, 1e-6)
+    assert_bits(ctx.download(xd, np.float32, dim + 1)[1:], want)
+
+
 def test_swiglu_quant(ctx, orc):
     rng = np.random.default_rng(4)
     dim = 5888
@@ -328,6 +341,14 @@ def test_attention(ctx, orc, case, heads):
     assert_bits(ctx.download(od, np.float32, nh * hd), want)
     assert_bits(ctx.download(kcd, np.float32, kc.size), kc2)
     assert_bits(ctx.download(vcd, np.float32, vc.size), vc2)
+
+
+# the combine's waves: head dims below and past a wave's 64, chunk counts at the edges of its 16-chunk
+# batches and past the 64 chunks a wave's lanes hold
+@pytest.mark.parametrize("heads", [(4, 4, 4), (8, 2, 80)])
+@pytest.mark.parametrize("pos", [63, 64 * 15, 64 * 16, 64 * 17 - 1, 64 * 64 - 1, 64 * 80 + 5])
+def test_attention_combine_edges(ctx, orc, heads, pos):
+    test_attention(ctx, orc, (pos, pos + 1), heads)
 
 
 def test_attention_context_overflow(ctx):
