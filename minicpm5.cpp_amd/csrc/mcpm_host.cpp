@@ -163,16 +163,6 @@ bool is_q8k_type(const mcpm_tensor* w) {
   return w && (w->t.type == MCPM_TYPE_Q4_K || w->t.type == MCPM_TYPE_Q6_K);
 }
 
-int set_state(mcpm_ctx* ctx, int token, int pos) {
-  ctx->h_state->token = token;
-  ctx->h_state->pos = pos;
-  ctx->h_state->step = 0;
-  ctx->h_state->n_out = 0;
-  MCPM_HIP(hipMemcpyAsync(ctx->d_state, ctx->h_state, sizeof(StepState), hipMemcpyHostToDevice, ctx->stream));
-  MCPM_HIP(hipStreamSynchronize(ctx->stream));
-  return MCPM_OK;
-}
-
 GemvArgs single_region(const mcpm_tensor* w, float* out, int rows, int cols) {
   GemvArgs a{};
   a.reg[0] = GemvRegion{view_of(w->t), out, 0, rows};
@@ -236,8 +226,6 @@ int mcpm_init(int device, mcpm_ctx** out) {
   c->n_cu = prop.multiProcessorCount;
   c->name = prop.gcnArchName;
   e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&c->d_state, sizeof(StepState));
-  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&c->h_state), sizeof(StepState), hipHostMallocDefault);
   if (e == hipSuccess) e = hipMalloc(&c->d_rope, 512 * sizeof(float2));
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&c->h_rope), 512 * sizeof(float2), hipHostMallocDefault);
   if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -258,8 +246,6 @@ void mcpm_destroy(mcpm_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->d_state) (void)hipFree(c->d_state);
-  if (c->h_state) (void)hipHostFree(c->h_state);
   if (c->d_rope) (void)hipFree(c->d_rope);
   if (c->h_rope) (void)hipHostFree(c->h_rope);
   if (c->d_attn_part) (void)hipFree(c->d_attn_part);
@@ -559,9 +545,15 @@ int mcpm_swiglu_and_quantize_q8k(mcpm_ctx* c, void* out, const float* gate, cons
 int mcpm_apply_rope(mcpm_ctx* c, float* vec, int pos, int n_heads, int head_dim, float base) {
   if (!c || !vec || n_heads <= 0 || head_dim <= 0 || head_dim % 2 || head_dim / 2 > c->rope_cap || pos < 0)
     return fail(MCPM_ERR_ARG, "mcpm_apply_rope: bad argument");
-  rope_row(pos, head_dim, base, c->h_rope);
-  MCPM_HIP(hipMemcpyAsync(c->d_rope, c->h_rope, sizeof(float2) * (head_dim / 2), hipMemcpyHostToDevice, c->stream));
-  MCPM_HIP(launch_rope(vec, c->d_rope, n_heads, head_dim, c->stream));
+  RopeRow row;
+  if (head_dim / 2 <= RopeRow::MAX) {
+    rope_row(pos, head_dim, base, row.v);
+    MCPM_HIP(launch_rope(vec, row, nullptr, n_heads, head_dim, c->stream));
+  } else {
+    rope_row(pos, head_dim, base, c->h_rope);
+    MCPM_HIP(hipMemcpyAsync(c->d_rope, c->h_rope, sizeof(float2) * (head_dim / 2), hipMemcpyHostToDevice, c->stream));
+    MCPM_HIP(launch_rope(vec, row, c->d_rope, n_heads, head_dim, c->stream));
+  }
   MCPM_HIP(hipStreamSynchronize(c->stream));
   return MCPM_OK;
 }
@@ -577,14 +569,12 @@ int mcpm_execute_attention(mcpm_ctx* c, float* out, const float* q, const float*
   const int max_chunks = (max_seq_len + ATTN_CHUNK - 1) / ATTN_CHUNK;
   int rc = ensure_attn_scratch(c, static_cast<size_t>(n_heads) * max_chunks * (2 + head_dim));
   if (rc) return rc;
-  rc = set_state(c, 0, pos);
-  if (rc) return rc;
-  const int kvd = n_kv_heads * head_dim;
-  const int* st = reinterpret_cast<const int*>(c->d_state);
-  MCPM_HIP(launch_kv_append(k_cur, v_cur, k_cache, v_cache, st, kvd, c->stream));
+  // the position goes in the launches' arguments: no copy and no wait comes before them
+  MCPM_HIP(launch_kv_append(k_cur, v_cur, k_cache, v_cache, pos, n_kv_heads * head_dim, c->stream));
   const AttnPart part = attn_part_of(c->d_attn_part, n_heads, max_chunks, head_dim);
-  MCPM_HIP(launch_attention(q, k_cache, v_cache, st, n_heads, n_kv_heads, head_dim, max_chunks, part, c->stream));
-  MCPM_HIP(launch_attn_combine(part, st, n_heads, head_dim, max_chunks, out, c->stream));
+  MCPM_HIP(launch_attention(q, k_cache, v_cache, nullptr, n_heads, n_kv_heads, head_dim, max_chunks, part, c->stream,
+                            pos));
+  MCPM_HIP(launch_attn_combine(part, nullptr, n_heads, head_dim, max_chunks, out, c->stream, pos));
   MCPM_HIP(hipStreamSynchronize(c->stream));
   return MCPM_OK;
 }
@@ -597,9 +587,7 @@ int mcpm_get_embedding(mcpm_ctx* c, float* out, const mcpm_tensor* e, int token)
     return fail(MCPM_ERR_UNSUPPORTED, "get_embedding implemented for Q4_K and Q6_K only");
   }
   if (token < 0 || token >= e->t.rows) return fail(MCPM_ERR_ARG, "mcpm_get_embedding: token out of range");
-  int rc = set_state(c, token, 0);
-  if (rc) return rc;
-  MCPM_HIP(launch_embedding(view_of(e->t), reinterpret_cast<const int*>(c->d_state), dim, out, c->stream));
+  MCPM_HIP(launch_embedding(view_of(e->t), nullptr, dim, out, c->stream, nullptr, token));
   return MCPM_OK;
 }
 

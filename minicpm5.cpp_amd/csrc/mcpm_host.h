@@ -12,9 +12,7 @@ struct mcpm_ctx {
   std::string name;
   hipStream_t stream = nullptr;
   // per-op scratch, grown on demand
-  mcpm::StepState* d_state = nullptr;
-  mcpm::StepState* h_state = nullptr;  // pinned
-  float2* d_rope = nullptr;            // one (cos, sin) row
+  float2* d_rope = nullptr;            // one (cos, sin) row longer than a kernel argument holds
   float2* h_rope = nullptr;            // pinned
   int rope_cap = 0;
   float* d_attn_part = nullptr;

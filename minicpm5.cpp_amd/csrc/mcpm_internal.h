@@ -316,11 +316,18 @@ hipError_t launch_quantize_q8k(const float* x, const float* gamma, float eps, in
                                hipStream_t s);
 hipError_t launch_rmsnorm(const float* x, const float* w, float eps, int dim, float* out, hipStream_t s);
 hipError_t launch_swiglu_quant(const float* g, const float* u, int dim, BlockQ8K* out, hipStream_t s);
-hipError_t launch_rope(float* vec, const float2* cs, int n_heads, int head_dim, hipStream_t s);
-hipError_t launch_kv_append(const float* k, const float* v, float* kc, float* vc, const int* state, int kvd,
-                            hipStream_t s);
+// One position's (cos, sin) pairs, as a kernel argument.
+struct RopeRow {
+  static constexpr int MAX = 64;
+  float2 v[MAX];
+};
+hipError_t launch_rope(float* vec, const RopeRow& row, const float2* device, int n_heads, int head_dim,
+                       hipStream_t s);
+hipError_t launch_kv_append(const float* k, const float* v, float* kc, float* vc, int pos, int kvd, hipStream_t s);
+// pos >= 0 (here and in launch_attn_combine): the position, in place of the step state's.
 hipError_t launch_attention(const float* q, const float* kc, const float* vc, const int* state, int n_heads,
-                            int n_kv_heads, int head_dim, int max_chunks, const AttnPart& part, hipStream_t s);
+                            int n_kv_heads, int head_dim, int max_chunks, const AttnPart& part, hipStream_t s,
+                            int pos = -1);
 // Decode attention for contexts of at most ATTN_Q8K_MAX_CHUNKS chunks (512
 // positions), head_dim 64, one work group per kv head, its output combined and quantized ties-even into Q8_K blocks
 // (for the O projection); shapes whose query group covers whole blocks.
@@ -334,7 +341,7 @@ inline bool attn_q8k_fits(int n_heads, int n_kv_heads, int head_dim) {
 hipError_t launch_attention_q8k(const float* q, const float* kc, const float* vc, const int* state, int n_heads,
                                 int n_kv_heads, int head_dim, BlockQ8K* out, unsigned* err, hipStream_t s);
 hipError_t launch_attn_combine(const AttnPart& part, const int* state, int n_heads, int head_dim, int max_chunks,
-                               float* out, hipStream_t s);
+                               float* out, hipStream_t s, int pos = -1);
 
 // ---- prefill (batched prompt tokens; csrc/mcpm_prefill.hip) ----
 // Per-token Q8_K activations: fp16 codes [t][dim], d [t][dim/256], fp16
@@ -368,8 +375,9 @@ hipError_t launch_attention_batch(const float* q, const float* kc, const float* 
 hipError_t launch_quant_batch_attn(const AttnPart& part, size_t tok_stride_o, size_t tok_stride_mz, int pos0,
                                    int n_tok, int n_heads, int head_dim, int max_chunks, QuantBatch q, hipStream_t s);
 // epoch (optional): advanced by one (the tags of the token's XCD records).
+// token >= 0: that row, in place of the step state's token.
 hipError_t launch_embedding(const WView& w, const int* state, int dim, float* out, hipStream_t s,
-                            unsigned* epoch = nullptr);
+                            unsigned* epoch = nullptr, int token = -1);
 hipError_t launch_dequant_rows(const WView& w, int row0, int n_rows, int cols, float* out, hipStream_t s);
 hipError_t launch_gemv_f32(const float* w, const float* x, float* out, int rows, int cols, hipStream_t s);
 hipError_t launch_stream_read(const void* src, size_t bytes, int grid, uint32_t* out, hipStream_t s);

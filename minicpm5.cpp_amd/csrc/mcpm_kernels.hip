@@ -145,34 +145,40 @@ hipError_t launch_swiglu_quant(const float* g, const float* u, int dim, BlockQ8K
   return hipGetLastError();
 }
 
-// apply_rope for every head with a host-built (cos, sin) row for pos.
-__global__ void k_rope(float* __restrict__ vec, const float2* __restrict__ cs, int n_pairs, int half_hd) {
+// apply_rope for every head with a host-built (cos, sin) row for pos, held in
+// the kernel's arguments: no copy to the device comes before the launch.
+// (device, when not null, holds the row instead: rows past RopeRow::MAX pairs.)
+__global__ void k_rope(float* __restrict__ vec, const RopeRow row, const float2* __restrict__ device, int n_pairs,
+                       int half_hd) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n_pairs) return;
-  const float2 c = cs[p % half_hd];
+  const float2 c = device ? device[p % half_hd] : row.v[p % half_hd];
   const float v0 = vec[2 * p], v1 = vec[2 * p + 1];
   vec[2 * p] = v0 * c.x - v1 * c.y;
   vec[2 * p + 1] = v0 * c.y + v1 * c.x;
 }
 
-hipError_t launch_rope(float* vec, const float2* cs, int n_heads, int head_dim, hipStream_t s) {
+hipError_t launch_rope(float* vec, const RopeRow& row, const float2* device, int n_heads, int head_dim,
+                       hipStream_t s) {
+  if (!device && head_dim / 2 > RopeRow::MAX) return hipErrorInvalidValue;
   const int n_pairs = n_heads * head_dim / 2;
-  hipLaunchKernelGGL(k_rope, dim3((n_pairs + 255) / 256), dim3(256), 0, s, vec, cs, n_pairs, head_dim / 2);
+  hipLaunchKernelGGL(k_rope, dim3((n_pairs + 255) / 256), dim3(256), 0, s, vec, row, device, n_pairs,
+                     head_dim / 2);
   return hipGetLastError();
 }
 
 __global__ void k_kv_append(const float* __restrict__ k, const float* __restrict__ v, float* __restrict__ kc,
-                            float* __restrict__ vc, const int* __restrict__ state, int kvd) {
+                            float* __restrict__ vc, int pos, int kvd) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= kvd) return;
-  const size_t pos = static_cast<size_t>(state[1]);
-  kc[pos * kvd + i] = k[i];
-  vc[pos * kvd + i] = v[i];
+  const size_t o = static_cast<size_t>(pos) * kvd + i;
+  kc[o] = k[i];
+  vc[o] = v[i];
 }
 
-hipError_t launch_kv_append(const float* k, const float* v, float* kc, float* vc, const int* state, int kvd,
+hipError_t launch_kv_append(const float* k, const float* v, float* kc, float* vc, int pos, int kvd,
                             hipStream_t s) {
-  hipLaunchKernelGGL(k_kv_append, dim3((kvd + 255) / 256), dim3(256), 0, s, k, v, kc, vc, state, kvd);
+  hipLaunchKernelGGL(k_kv_append, dim3((kvd + 255) / 256), dim3(256), 0, s, k, v, kc, vc, pos, kvd);
   return hipGetLastError();
 }
 
@@ -309,19 +315,10 @@ __global__ void __launch_bounds__(256) k_attention(const float* __restrict__ q, 
                                                    const float* __restrict__ vc, const int* __restrict__ state,
                                                    int n_heads, int n_kv_heads, int hd, int max_chunks,
                                                    float* __restrict__ part_o, float2* __restrict__ part_mz,
-                                                   int pos0, size_t tok_q, size_t tok_o, size_t tok_mz) {
+                                                   int pos) {
   __shared__ __attribute__((aligned(16))) float lds[AttnLds<HDM>::bytes / sizeof(float)];
-  // decode: the position from the step state; prefill (pos0 >= 0): token
-  // blockIdx.z at position pos0 + z, with its own q and partials
-  int T;
-  if (pos0 >= 0) {
-    T = pos0 + static_cast<int>(blockIdx.z) + 1;
-    q += blockIdx.z * tok_q;
-    part_o += blockIdx.z * tok_o;
-    part_mz += blockIdx.z * tok_mz;
-  } else {
-    T = state[1] + 1;
-  }
+  // the position: given (pos >= 0), or the step state's
+  const int T = (pos >= 0 ? pos : state[1]) + 1;
   AttnRegs<HDM / 16> R;
   attn_split<HDM, false, WL>(q, kc, vc, T, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y), n_heads,
                          n_kv_heads, hd, max_chunks, part_o, part_mz, AttnLds<HDM>(lds), R, false);
@@ -608,9 +605,9 @@ constexpr int COMBINE_BATCH = 16;
 
 __global__ void __launch_bounds__(64) k_attn_combine(const float* __restrict__ part_o,
                                                      const float2* __restrict__ part_mz,
-                                                     const int* __restrict__ state, int hd, int max_chunks,
+                                                     const int* __restrict__ state, int pos, int hd, int max_chunks,
                                                      float* __restrict__ out) {
-  const int nch = state[1] / ATTN_CHUNK + 1;
+  const int nch = (pos >= 0 ? pos : state[1]) / ATTN_CHUNK + 1;
   const int h = blockIdx.x, lane = threadIdx.x, d = blockIdx.y * 64 + lane;
   const float2* mz = part_mz + static_cast<size_t>(h) * max_chunks;
   // lanes past the head's dims repeat its last one (unused)
@@ -645,18 +642,20 @@ __global__ void __launch_bounds__(64) k_attn_combine(const float* __restrict__ p
 }
 
 hipError_t launch_attention(const float* q, const float* kc, const float* vc, const int* state, int n_heads,
-                            int n_kv_heads, int head_dim, int max_chunks, const AttnPart& part, hipStream_t s) {
+                            int n_kv_heads, int head_dim, int max_chunks, const AttnPart& part, hipStream_t s,
+                            int pos) {
   if (head_dim <= 0 || head_dim > 128 || head_dim % 4 || n_heads % n_kv_heads ||
       n_heads / n_kv_heads > ATTN_MAX_GROUP)
     return hipErrorInvalidValue;
-  const dim3 grid(n_kv_heads, attn_max_splits(1, max_chunks));
+  // a given position needs its own splits only; the step state's may be any
+  const dim3 grid(n_kv_heads, pos >= 0 ? attn_splits(pos / ATTN_CHUNK + 1) : attn_max_splits(1, max_chunks));
   if (head_dim <= 64)
     launch_kernel(head_dim == 64 ? k_attention<64, true> : k_attention<64, false>, grid, dim3(256), 0, s, q, kc, vc,
                   state, n_heads, n_kv_heads, head_dim,
-                  max_chunks, part.o, part.mz, -1, size_t{0}, size_t{0}, size_t{0});
+                  max_chunks, part.o, part.mz, pos);
   else
     launch_kernel(k_attention<128, false>, grid, dim3(256), 0, s, q, kc, vc, state, n_heads, n_kv_heads, head_dim,
-                  max_chunks, part.o, part.mz, -1, size_t{0}, size_t{0}, size_t{0});
+                  max_chunks, part.o, part.mz, pos);
   return hipGetLastError();
 }
 
@@ -701,9 +700,9 @@ hipError_t launch_attention_batch(const float* q, const float* kc, const float* 
 }
 
 hipError_t launch_attn_combine(const AttnPart& part, const int* state, int n_heads, int head_dim, int max_chunks,
-                               float* out, hipStream_t s) {
+                               float* out, hipStream_t s, int pos) {
   hipLaunchKernelGGL(k_attn_combine, dim3(n_heads, (head_dim + 63) / 64), dim3(64), 0, s, part.o, part.mz, state,
-                     head_dim, max_chunks, out);
+                     pos, head_dim, max_chunks, out);
   return hipGetLastError();
 }
 
@@ -730,20 +729,20 @@ hipError_t launch_dequant_rows(const WView& w, int row0, int n_rows, int cols, f
   return hipGetLastError();
 }
 
-// get_embedding: row `token` (from the step state) dequantized to x; one
+// get_embedding: row `token` (when negative: the step state's) dequantized to x; one
 // work group per 256-value block, one value per thread.  epoch (optional):
 // advanced by one, by one thread.
-__global__ void __launch_bounds__(256) k_embedding(const WView w, const int* __restrict__ state, int dim,
-                                                   float* __restrict__ out, unsigned* epoch) {
-  const int token = state[0];
+__global__ void __launch_bounds__(256) k_embedding(const WView w, const int* __restrict__ state, int token,
+                                                   int dim, float* __restrict__ out, unsigned* epoch) {
+  if (token < 0) token = state[0];
   const int i = blockIdx.x * QK_K + threadIdx.x;
   if (i < dim) out[i] = dequant_value(w, token, blockIdx.x, threadIdx.x);
   if (epoch && i == 0) epoch[0] = epoch[0] + 1u;
 }
 
 hipError_t launch_embedding(const WView& w, const int* state, int dim, float* out, hipStream_t s,
-                            unsigned* epoch) {
-  hipLaunchKernelGGL(k_embedding, dim3((dim + QK_K - 1) / QK_K), dim3(QK_K), 0, s, w, state, dim, out, epoch);
+                            unsigned* epoch, int token) {
+  hipLaunchKernelGGL(k_embedding, dim3((dim + QK_K - 1) / QK_K), dim3(QK_K), 0, s, w, state, token, dim, out, epoch);
   return hipGetLastError();
 }
 

@@ -63,18 +63,11 @@ extern "C" int mcpm_execute_attention_noalloc(mcpm_ctx* c, float* out, const flo
                                   std::to_string(kScratchFloats));
   float* base = (c->device >= 0 && c->device < kMaxDevices) ? g_scratch[c->device] : nullptr;
   if (!base) return fail(MCPM_ERR_CONTEXT, "mcpm_execute_attention_noalloc: scratch not set up for this device");
-  // the position, through the context's pinned staging (allocated at mcpm_init)
-  c->h_state->token = 0;
-  c->h_state->pos = pos;
-  c->h_state->step = 0;
-  c->h_state->n_out = 0;
-  MCPM_HIP(hipMemcpyAsync(c->d_state, c->h_state, sizeof(StepState), hipMemcpyHostToDevice, c->stream));
-  const int kvd = n_kv_heads * head_dim;
-  const int* st = reinterpret_cast<const int*>(c->d_state);
-  MCPM_HIP(launch_kv_append(k_cur, v_cur, k_cache, v_cache, st, kvd, c->stream));
+  MCPM_HIP(launch_kv_append(k_cur, v_cur, k_cache, v_cache, pos, n_kv_heads * head_dim, c->stream));
   const AttnPart part = attn_part_of(base, n_heads, max_chunks, head_dim);
-  MCPM_HIP(launch_attention(q, k_cache, v_cache, st, n_heads, n_kv_heads, head_dim, max_chunks, part, c->stream));
-  MCPM_HIP(launch_attn_combine(part, st, n_heads, head_dim, max_chunks, out, c->stream));
+  MCPM_HIP(launch_attention(q, k_cache, v_cache, nullptr, n_heads, n_kv_heads, head_dim, max_chunks, part, c->stream,
+                            pos));
+  MCPM_HIP(launch_attn_combine(part, nullptr, n_heads, head_dim, max_chunks, out, c->stream, pos));
   MCPM_HIP(hipStreamSynchronize(c->stream));
   return MCPM_OK;
 }
