@@ -701,9 +701,12 @@ int ensure_prefill(mcpm_engine* e, int cap) {
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.g), n * c.ffn * 4);
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.u), n * c.ffn * 4);
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.part), n * c.n_heads * e->max_chunks * (c.head_dim + 2) * 4);
-  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xh), n * kmax * 2);
-  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xd), n * (kmax / QK_K) * 4);
-  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xbs), n * (kmax / QK_K) * 16 * 2);
+  // quantized activations: whole tiles of 16 tokens, and the 16 bytes a GEMM
+  // lane may read past the last bsums
+  const size_t nt = (n + 15) / 16 * 16;
+  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xh), nt * kmax * 2);
+  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xd), nt * (kmax / QK_K) * 4);
+  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xbs), nt * (kmax / QK_K) * 16 * 2 + 16);
   if (rc) {
     free_prefill(b);
     return rc;

@@ -344,8 +344,9 @@ hipError_t launch_attn_combine(const AttnPart& part, const int* state, int n_hea
                                float* out, hipStream_t s, int pos = -1);
 
 // ---- prefill (batched prompt tokens; csrc/mcpm_prefill.hip) ----
-// Per-token Q8_K activations: fp16 codes [t][dim], d [t][dim/256], fp16
-// bsums [t][dim/256][16].
+// Per-token Q8_K activations in tiles of 16 tokens (the last one whole): fp16
+// codes in the GEMM's operand order, d [tile][dim/256][16], fp16 bsums
+// [tile][dim/256][16][16] and 16 readable bytes after them.
 struct QuantBatch {
   _Float16* xh;
   float* xd;
@@ -363,7 +364,7 @@ struct GemmRope {
   int head_dim, pos0;
 };
 // w2 / rows2 / out2 / ld_out2: a second matrix of w's type on the same
-// activations in the same launch (rows % 64 == 0).
+// activations in the same launch.
 hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const QuantBatch& q, float* out, int ld_out,
                            bool add, hipStream_t s, const WView* w2 = nullptr, int rows2 = 0, float* out2 = nullptr,
                            int ld_out2 = 0, const GemmRope* rope = nullptr, bool swiglu = false);

@@ -12,7 +12,7 @@
 //    order, Q4_K's min chain, and ((a0+a4)+(a2+a6))+((a1+a5)+(a3+a7));
 //  * isum[m] for 16 rows x 16 tokens is one v_mfma_f32_16x16x32_f16: K runs
 //    over lane m's 32 bytes (8 sub-blocks x 4) with A = sub-block scale x
-//    weight code and B = activation code.  Every product is an integer of at
+//    weight code (over 64) and activation code (times 64).  Every product is an integer of at
 //    most 2048 in magnitude (exact in fp16) and every sum stays below 2^24
 //    (exact in fp32), so the MFMA result is isum[m] itself.  Q4_K: sc*q <= 945.
 //    Q6_K: the reference sums sc*q*x over lane m's bytes (q in 0..63) and
@@ -26,7 +26,7 @@
 //    nearest even, as the reference's int32 -> float conversion of the same
 //    integer does.
 //  * Q4_K's min sum (sum over sub-blocks of mn * pair-sum of bsums) is one
-//    more MFMA: A = mn[k/2] for k < 16, B = bsums[k].
+//    more MFMA: mn[k/2] for k < 16 against bsums[k].
 // Attention per token is the decode kernel at that token's position.
 #include <algorithm>
 #include <cstdio>
@@ -57,12 +57,45 @@ __global__ void __launch_bounds__(256) k_embed_batch(const WView w, const int* _
 // i < n_valid and 0 beyond, then ties-away (decode's down prologue).
 constexpr int QB_SWIGLU = 100;
 
+// The quantized activations in the order the GEMM's MFMA operands want them,
+// in tiles of 16 tokens: codes [tile][block][lane group m][K-half g][token of
+// the tile][8 halves], the 8 halves being elements 64g + 4m .. +3 and 64g + 32
+// + 4m .. +3 of the block, each code times 64 (exact in fp16; the weights'
+// operands are divided by 64); d [tile][block][token]; bsums
+// [tile][block][token][16].  A GEMM wave then reads a lane group's whole
+// operand (64 lanes x 16 bytes) as one run of 1 KiB, with no staging in LDS.
+// lane: the block's values 4*lane .. +3.
+__device__ __forceinline__ void store_codes(int t, int nb, int b, int lane, uint32_t packed, float d, int gsum,
+                                            _Float16* __restrict__ xh, float* __restrict__ xd,
+                                            _Float16* __restrict__ xbs) {
+  typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+  const size_t tb = static_cast<size_t>(t >> 4) * nb + b;
+  const int c = t & 15, m = lane & 7, half = (lane >> 3) & 1, g = lane >> 4;
+  h4 hv;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    hv[k] = static_cast<_Float16>(64.0f * static_cast<float>(static_cast<int8_t>((packed >> (8 * k)) & 0xffu)));
+  *reinterpret_cast<h4*>(xh + (tb * 8 + m) * 512 + (16 * g + c) * 8 + 4 * half) = hv;
+  if ((lane & 3) == 0) xbs[(tb * 16 + c) * 16 + (lane >> 2)] = static_cast<_Float16>(gsum);
+  if (lane == 0) xd[tb * 16 + c] = d;
+}
+
+// The token of a quantization work group: a tile's 16 tokens share cache lines
+// of the operand layout, so they go to one XCD (work group b runs on XCD b %
+// 8), whose L2 puts the lines together.
+__device__ __forceinline__ int quant_token(unsigned b) {
+  const int xcd = static_cast<int>(b & 7), j = static_cast<int>(b >> 3);
+  return 16 * (xcd + 8 * (j >> 4)) + (j & 15);
+}
+static dim3 quant_grid(int n_tok) { return dim3(128 * ((n_tok + 127) / 128)); }
+
 __global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x, const float* __restrict__ u,
                                                      int ld_x, const float* __restrict__ gamma, float eps, int dim,
-                                                     int n_valid, int mode, _Float16* __restrict__ xh,
+                                                     int n_valid, int mode, int n_tok, _Float16* __restrict__ xh,
                                                      float* __restrict__ xd, _Float16* __restrict__ xbs) {
   __shared__ float red[260];
-  const int t = blockIdx.x;
+  const int t = quant_token(blockIdx.x);
+  if (t >= n_tok) return;  // uniform, before any barrier
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float* xt = x + static_cast<size_t>(t) * ld_x;
   const float* ut = u ? u + static_cast<size_t>(t) * ld_x : nullptr;
@@ -93,12 +126,7 @@ __global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x
     float d;
     int gsum;
     quant_block_wave(v, away, packed, d, gsum);
-    _Float16* o = xh + static_cast<size_t>(t) * dim + b * QK_K + 4 * lane;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      o[k] = static_cast<_Float16>(static_cast<float>(static_cast<int8_t>((packed >> (8 * k)) & 0xffu)));
-    if ((lane & 3) == 0) xbs[(static_cast<size_t>(t) * nb + b) * 16 + (lane >> 2)] = static_cast<_Float16>(gsum);
-    if (lane == 0) xd[static_cast<size_t>(t) * nb + b] = d;
+    store_codes(t, nb, b, lane, packed, d, gsum, xh, xd, xbs);
   }
 }
 
@@ -111,11 +139,12 @@ __global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x
 template <int MAXB>
 __global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__ x, const float* __restrict__ u,
                                                        int ld_x, const float* __restrict__ gamma, float eps, int dim,
-                                                       int n_valid, int mode, _Float16* __restrict__ xh,
+                                                       int n_valid, int mode, int n_tok, _Float16* __restrict__ xh,
                                                        float* __restrict__ xd, _Float16* __restrict__ xbs) {
   __shared__ float red[260];
   __shared__ __attribute__((aligned(16))) float sx[4 * MAXB * QK_K];
-  const int t = blockIdx.x;
+  const int t = quant_token(blockIdx.x);
+  if (t >= n_tok) return;  // uniform, before any barrier
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const float* xt = x + static_cast<size_t>(t) * ld_x;
   const float* ut = u ? u + static_cast<size_t>(t) * ld_x : nullptr;
@@ -173,15 +202,7 @@ __global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__
     float d;
     int gsum;
     quant_block_wave(v, away, packed, d, gsum);
-    _Float16* o = xh + static_cast<size_t>(t) * dim + b * QK_K + 4 * lane;
-    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-    h4 hv;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      hv[k] = static_cast<_Float16>(static_cast<float>(static_cast<int8_t>((packed >> (8 * k)) & 0xffu)));
-    *reinterpret_cast<h4*>(o) = hv;
-    if ((lane & 3) == 0) xbs[(static_cast<size_t>(t) * nb + b) * 16 + (lane >> 2)] = static_cast<_Float16>(gsum);
-    if (lane == 0) xd[static_cast<size_t>(t) * nb + b] = d;
+    store_codes(t, nb, b, lane, packed, d, gsum, xh, xd, xbs);
   }
 }
 
@@ -189,15 +210,15 @@ __global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__
 struct GemmArgs {
   WView w;
   int rows, nb, n_tok;
-  const _Float16* xh;   // [n_tok][nb*256] activation codes
-  const float* xd;      // [n_tok][nb] Q8_K d
-  const _Float16* xbs;  // [n_tok][nb][16] bsums
+  // quantized activations in store_codes' layout (whole tiles of 16 tokens)
+  const _Float16* xh;
+  const float* xd;
+  const _Float16* xbs;
   float* out;           // out[t*ld_out + r]
   int ld_out;
   int add;              // 1: out += v (residual), 0: out = v
   // an optional second matrix of the same type and blocks per row on the
-  // same activations (rows2 > 0, rows a multiple of 64): the launch's rows
-  // rows .. rows+rows2-1 are its rows, written to out2 (row stride ld_out2)
+  // same activations (rows2 > 0), written to out2 (row stride ld_out2)
   WView w2;
   int rows2;
   float* out2;
@@ -207,9 +228,9 @@ struct GemmArgs {
   // position pos0 + t, table rows of rope_hd/2 (cos, sin) pairs)
   const float2* rope;
   int rope_hd, pos0;
-  // swiglu: the two matrices are gate and up (rows2 == rows, rows % 32 ==
-  // 0); a work group takes 32 rows of each (waves 0, 1: gate; 2, 3: up) and
-  // writes h = silu(gate)*up (decode's gate/up epilogue) to out
+  // swiglu: the two matrices are gate and up (rows2 == rows); a work group
+  // takes the same rows of both and writes h = silu(gate)*up (decode's
+  // gate/up epilogue) to out
   int swiglu;
 };
 
@@ -220,61 +241,65 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rsrc(const void* p) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), static_cast<short>(0), 0x7fffffff, 0x00020000);
 }
 
-// fp16 pair (1024 + byte) from bytes of t picked by sel (0x64 high bytes),
-// minus off: small integers, exact
-__device__ __forceinline__ h2 byte_pair_h(uint32_t t, uint32_t sel, h2 off) {
-  return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, t, sel)) - off;
+// fp16 pair (1024 + byte) of the bytes of t that sel picks
+__device__ __forceinline__ h2 byte_pair(uint32_t t, uint32_t sel) {
+  return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, t, sel));
 }
 constexpr uint32_t SEL01 = 0x04010400u, SEL23 = 0x04030402u;
 
-// Eight halves of lane m's A operand: the low (j < 4) and high (j >= 4)
-// K-halves, each four bytes of ta / tb times sa / sb, as (1024 + byte) * s +
-// m in one packed fma with m = -1024 * s, whose single rounding meets the
-// exact product byte * s.  Q4_K: s = sc <= 63 (m exact in fp16, byte * s <=
-// 945).  Q6_K: s = sc / 64 for signed sc (m = -16 * sc, |byte * sc| <= 1920,
-// so byte * sc / 64 is exact in fp16); its MFMA sums come out divided by 64,
-// exactly, and the chain's scale carries the 64 back.
-__device__ __forceinline__ h2 byte_pair_fma(uint32_t t, uint32_t sel, h2 s, h2 ms) {
-  return __builtin_elementwise_fma(__builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, t, sel)), s, ms);
-}
-__device__ __forceinline__ h8 a_operand_fma(uint32_t ta, uint32_t tb, h2 sa, h2 sb, h2 ma, h2 mb) {
-  const u32x4 r{h2bits(byte_pair_fma(ta, SEL01, sa, ma)), h2bits(byte_pair_fma(ta, SEL23, sa, ma)),
-                h2bits(byte_pair_fma(tb, SEL01, sb, mb)), h2bits(byte_pair_fma(tb, SEL23, sb, mb))};
+// Eight halves of a weight operand: the low (j < 4) and high (j >= 4)
+// K-halves, each four bytes of ta / tb times sa / sb, as (1024 + byte) * s + m
+// in one packed fma with m = -1024 * s, whose single rounding meets the exact
+// product byte * s.  s = sc / 64 over the field's power of two: Q4_K sc <= 63
+// (byte * sc <= 945), Q6_K signed sc (|byte * sc| <= 1920), so byte * sc / 64
+// is exact in fp16, and the activations' factor 64 makes every MFMA product
+// the integer code * scale * code.
+__device__ __forceinline__ h8 w_operand(uint32_t ta, uint32_t tb, h2 sa, h2 sb, h2 ma, h2 mb) {
+  const u32x4 r{h2bits(__builtin_elementwise_fma(byte_pair(ta, SEL01), sa, ma)),
+                h2bits(__builtin_elementwise_fma(byte_pair(ta, SEL23), sa, ma)),
+                h2bits(__builtin_elementwise_fma(byte_pair(tb, SEL01), sb, mb)),
+                h2bits(__builtin_elementwise_fma(byte_pair(tb, SEL23), sb, mb))};
   return __builtin_bit_cast(h8, r);
 }
 
-__device__ __forceinline__ h2 splat_h(int v) {
-  const _Float16 h = static_cast<_Float16>(static_cast<float>(v));
+__device__ __forceinline__ h2 splat2(float v) {
+  const _Float16 h = static_cast<_Float16>(v);
   return h2{h, h};
 }
 
-// A work group takes 64 rows (one 16-row tile per wave) x 16*NT tokens over
-// all blocks.  The tokens' activations of a block (codes, d, bsums) are
-// staged in LDS once for the four waves, double-buffered: block b+1's loads
-// are in flight while block b's MFMAs run.  MFMA operand
-// layout (v_mfma_f32_16x16x32_f16): lane l feeds A row l%16 and B column
-// l%16 with K = 8*(l/16) .. +7; D lane l register i is row 4*(l/16)+i,
-// column l%16.  With K index k = 4*s + i over sub-blocks s and bytes i,
-// lane l's K range is sub-blocks 2g and 2g+1 (g = l/16): element 64g + 4m + i
-// (low) and 64g + 32 + 4m + i (high) of the block for lane group m.
-template <int WT, int NT, int OCC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8))) k_gemm_q8k(const GemmArgs a) {
-  constexpr int TOK = 16 * NT;        // tokens of the work group's tile
-  constexpr int BROW = QK_K + 8;      // halves per token row of sB (padded: rows 132 dwords apart)
-  // halves per token of sBs.  Q4_K: the 16 bsums (rows 12 dwords apart).
-  // Q6_K: eight 16-byte records, record m = (bsums 2m, 2m+1 as an fp16
-  // pair, then zeros): lane group m's offset B operand read whole; a zero
-  // row after the tokens serves the lanes whose K entries are all zero.
-  constexpr int BSROW = WT == 0 ? 24 : 64;
-  constexpr int BSZERO = WT == 0 ? 0 : 64;
-  constexpr int PPT = TOK * 32 / 256; // 16-byte pieces of a block's codes per thread
-  __shared__ __attribute__((aligned(16))) _Float16 sB[2][TOK * BROW];
-  __shared__ float sXd[2][TOK];
-  __shared__ __attribute__((aligned(16))) _Float16 sBs[2][TOK * BSROW + BSZERO];
-  const int tid = threadIdx.x, wave = tid >> 6;
-  const int lane = tid & 63, g = lane >> 4, c16 = lane & 15;
-  const int n_rt = (a.rows + a.rows2 + 15) >> 4;
-  const int n_rg = (n_rt + 3) >> 2;
+// A work group of four waves takes 16*RT rows x 16*NT tokens over all blocks;
+// wave w takes lane groups 2w and 2w+1 of every block, whose chains over the
+// blocks no other lane group's touch, so the waves meet only at the end.
+// MFMA operand layout (v_mfma_f32_16x16x32_f16), activations as A, weights as
+// B: lane l feeds A row (token) l%16 and B column (weight row) l%16 with K =
+// 8*g .. +7, g = l/16; D lane l register i is token 4g+i, weight row l%16, so
+// the row whose scales a lane decodes is the row of its results.  With K index
+// k = 4*s + i over sub-blocks s and bytes i, a lane's K range is sub-blocks 2g
+// and 2g+1: elements 64g + 4m + i and 64g + 32 + 4m + i for lane group m.
+// What bounds it: one wave per lane-group pair (not per row tile) lets a weight
+// operand, whose build costs more than its MFMA, serve up to four token tiles
+// in the registers that two took (a wave's chains are 8 floats per result where
+// all lane groups in one wave need 32), and a short prompt's rows run on four
+// waves at once.  Against a work group of four row tiles x all lane groups with
+// activations staged in LDS (a barrier per block): 1023 tokens of the 2.4B
+// shape, gate/up 198 -> 131 us, down 171 -> 125, the prompt 23.8 -> 20.5 ms;
+// 44 tokens, down 30 -> 19 us, v 12.5 -> 9.2, the prompt 5.2 -> 4.0 ms.  Past
+// 64 tokens the activation operands' reads (16 TB/s from the L2s for gate/up)
+// bound it, for short prompts each wave's own chain of blocks (0.3 us a block
+// of Q6_K, 0.2 of Q4_K) and the first weights from HBM.
+// PF: blocks in flight (loads return in order, so weights and activations are
+// loaded equally far ahead).
+template <int WT, int RT, int NT, int PF>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_gemm_q8k(const GemmArgs a) {
+  constexpr int NM = (NT + 3) / 4;  // token tiles whose min chain and epilogue a wave takes: w, w+4, ...
+  __shared__ f32x4 s_acc[8 * NT * 64];  // one row tile's chains: [lane group][token tile][lane]
+  const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  // Row groups: the first matrix's, then the second's (swiglu: of RT/2 row
+  // tiles of both).
+  const int rpg = a.swiglu ? 8 * RT : 16 * RT;
+  const int n_rg1 = (a.rows + rpg - 1) / rpg;
+  const int n_rg = n_rg1 + (a.swiglu ? 0 : (a.rows2 + rpg - 1) / rpg);
   // XCD-aware tiles: work group b runs on XCD b % 8.  Of n_rg = 8q + r row
   // groups, XCD x takes rg = x + 8j (j < q) for every token tile (token
   // tiles outer, so the tile's activations serve its q row groups from one
@@ -282,7 +307,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8
   // token tile) items, so every XCD has the same work; each XCD's L2 keeps
   // about one eighth of the matrix for the whole launch.
   const int xcd = static_cast<int>(blockIdx.x) & 7, loc = static_cast<int>(blockIdx.x) >> 3;
-  const int n_tg = (a.n_tok + TOK - 1) / TOK;
+  const int n_tt = (a.n_tok + 15) >> 4;
+  const int n_tg = (n_tt + NT - 1) / NT;
   const int rq = n_rg >> 3, rr = n_rg & 7;
   const int share = (rr * n_tg + 7) >> 3;
   int rg, tg;
@@ -291,491 +317,289 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8
     tg = loc / rq;
   } else {
     const int li = xcd * share + (loc - rq * n_tg);
-    if (li >= rr * n_tg) return;  // uniform in the work group, before any barrier
+    if (loc - rq * n_tg >= share || li >= rr * n_tg) return;  // uniform in the work group, before any barrier
     rg = 8 * rq + li / n_tg;
     tg = li % n_tg;
   }
-  // the work group's matrix (its 64 rows lie in one: the first has a
-  // multiple of 64 rows)
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
-  const bool second = a.swiglu ? wv >= 2 : a.rows2 > 0 && 64 * rg >= a.rows;
-  const WView W = second ? a.w2 : a.w;
+  const bool second = rg >= n_rg1;
   const int rows = second ? a.rows2 : a.rows;
-  float* const out = second ? a.out2 : a.out;
-  const int ld_out = second ? a.ld_out2 : a.ld_out;
-  const int r0 = a.swiglu ? 32 * rg + 16 * (wv & 1) : (4 * rg + wave) * 16 - (second ? a.rows : 0), t0 = tg * TOK;
-  const bool live = r0 < rows;  // uniform in the wave: a wave past the rows only stages
-  const int ra = min(r0 + c16, rows - 1);  // A operand row of this lane
-  const int K = a.nb * QK_K;
-
-  // staging of block b: piece p = tid + 256k is 16 bytes (p % 32) of token
-  // p / 32's codes; thread t < TOK also takes token t's d, t < 2*TOK half of
-  // token t/2's bsums.  Tokens past the end re-read the last one (unused).
-  u32x4 pf[PPT], pbs;
-  float pxd = 0.0f;
-  // Every load of the block loop is a buffer load: the lane's byte offset is
-  // the same for every block (computed once here) and the block's part is a
-  // scalar offset, so the loop spends no vector instructions on addresses.
-  // (Every buffer here is far below 2 GB; indices are clamped as before.)
-  const __amdgpu_buffer_rsrc_t rxh = gemm_rsrc(a.xh), rxd = gemm_rsrc(a.xd), rxbs = gemm_rsrc(a.xbs);
-  uint32_t vo_pf[PPT];
-#pragma unroll
-  for (int k = 0; k < PPT; ++k) {
-    const int p = tid + 256 * k;
-    const uint32_t tk = static_cast<uint32_t>(min(t0 + p / 32, a.n_tok - 1));
-    vo_pf[k] = (tk * static_cast<uint32_t>(K) + static_cast<uint32_t>(p % 32) * 8) * 2;
-  }
-  // every thread loads (threads past the d and bsums slots re-read the
-  // last slot's, unused): no branch among the loads, so the waits for them
-  // count exactly
-  const int td = min(tid, TOK - 1), tb = min(tid, 2 * TOK - 1);
-  const uint32_t vo_xd = static_cast<uint32_t>(min(t0 + td, a.n_tok - 1)) * static_cast<uint32_t>(a.nb) * 4;
-  const uint32_t vo_xbs =
-      (static_cast<uint32_t>(min(t0 + tb / 2, a.n_tok - 1)) * static_cast<uint32_t>(a.nb) * 16 + (tb & 1) * 8) * 2;
-  auto fetch = [&](int b) {
-#pragma unroll
-    for (int k = 0; k < PPT; ++k)
-      pf[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rxh, vo_pf[k], b * QK_K * 2, 0));
-    pxd = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rxd, vo_xd, b * 4, 0));
-    pbs = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rxbs, vo_xbs, b * 32, 0));
+  // row tile rt's first row, and its matrix (swiglu: even tiles gate, odd up)
+  auto row0 = [&](int rt) {
+    return a.swiglu ? (rg * (RT / 2) + rt / 2) * 16 : ((second ? rg - n_rg1 : rg) * RT + rt) * 16;
   };
-  // sB keeps each token's 256 codes as 32 quads of 8 halves, quad 8g + m =
-  // elements 64g + 4m .. +3 and 64g + 32 + 4m .. +3 (the B operand of lane
-  // group m for the lanes of K-half g), stored at slot (8g + m) ^ sw(g) with
-  // sw = 0, 1, 1, 0 for g = 0..3: the lanes of one pass of 8-byte stores (16
-  // or 32) then write distinct banks, where unswapped quads 8 and 16 apart
-  // share them.  Piece k = p % 32 (elements 8k .. 8k+7, g = k/8, h =
-  // (k/4)%2, m = 2*(k%4)) goes to half h of quads m, m+1.
-  auto stash = [&](int buf) {
+  const WView& W0 = second ? a.w2 : a.w;
+  const WView& W1 = second || a.swiglu ? a.w2 : a.w;
+  const uint32_t rows16 = static_cast<uint32_t>(rows) * 16;
+
+  // Every load of the block loop is a buffer load whose lane offset is fixed
+  // here and whose block offset is a scalar.  Rows and token tiles past the
+  // end read the last one; their results are not stored.
+  struct WRaw {
+    // Q4_K: d, dmin and scales; lane groups 2w and 2w+1 of chunk 2g + w/2.
+    // Q6_K: scales 4g .. 4g+3, scales 4w .. 4w+3, d; ql of both 32-byte
+    // halves and qh of lane groups 2w, 2w+1.
+    u32x4 hdr;
+    u32x2 q[WT == 0 ? 1 : 3];
+  };
+  const __amdgpu_buffer_rsrc_t p00 = gemm_rsrc(W0.p0), p01 = gemm_rsrc(W1.p0), p10 = gemm_rsrc(W0.p1),
+                               p11 = gemm_rsrc(W1.p1), p20 = gemm_rsrc(W0.p2), p21 = gemm_rsrc(W1.p2),
+                               p30 = gemm_rsrc(W0.p3), p31 = gemm_rsrc(W1.p3);
+  uint32_t vr[RT];
 #pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-      const int p = tid + 256 * k;
-      const int pk = p % 32, gq = pk >> 3, hq = (pk >> 2) & 1, mq = 2 * (pk & 3), sw = (gq ^ (gq >> 1)) & 1;
-      _Float16* row = &sB[buf][(p / 32) * BROW + 4 * hq];
-      *reinterpret_cast<uint2*>(row + ((8 * gq + mq) ^ sw) * 8) = uint2{pf[k].x, pf[k].y};
-      *reinterpret_cast<uint2*>(row + ((8 * gq + mq + 1) ^ sw) * 8) = uint2{pf[k].z, pf[k].w};
-    }
-    if (tid < TOK) sXd[buf][tid] = pxd;
-    if (tid < 2 * TOK) {
+  for (int rt = 0; rt < RT; ++rt) vr[rt] = static_cast<uint32_t>(min(row0(rt) + c16, rows - 1));
+  const uint32_t w8 = 8u * static_cast<uint32_t>(w & 1);
+  auto load_w = [&](WRaw (&r)[RT], int b) {
+    const uint32_t ub = static_cast<uint32_t>(b);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const bool o = rt & 1;
       if constexpr (WT == 0) {
-        *reinterpret_cast<u32x4*>(&sBs[buf][(tid / 2) * BSROW + (tid & 1) * 8]) = pbs;
+        r[rt].hdr = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(o ? p11 : p10, vr[rt] * 16, ub * rows16, 0));
+        r[rt].q[0] = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(o ? p01 : p00, vr[rt] * 16 + 2 * g * rows16 + w8,
+                                                        (ub * 8 + static_cast<uint32_t>(w >> 1)) * rows16, 0));
       } else {
-        const uint32_t pw[4] = {pbs.x, pbs.y, pbs.z, pbs.w};
+        const uint32_t h = static_cast<uint32_t>(g >> 1);
+        r[rt].hdr.x = __builtin_amdgcn_raw_buffer_load_b32(o ? p21 : p20, vr[rt] * 16 + 4 * g, ub * rows16, 0);
+        r[rt].hdr.y = __builtin_amdgcn_raw_buffer_load_b32(o ? p21 : p20, vr[rt] * 16 + 4 * w, ub * rows16, 0);
+        r[rt].hdr.z = __builtin_amdgcn_raw_buffer_load_b16(o ? p31 : p30, vr[rt] * 2, ub * static_cast<uint32_t>(rows) * 2, 0);
+        const uint32_t ql = vr[rt] * 16 + 4 * h * rows16 + w8;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          *reinterpret_cast<uint32_t*>(&sBs[buf][(tid / 2) * BSROW + (4 * (tid & 1) + j) * 8]) = pw[j];
+        for (int k = 0; k < 2; ++k)
+          r[rt].q[k] = __builtin_bit_cast(
+              u32x2, __builtin_amdgcn_raw_buffer_load_b64(o ? p01 : p00, ql, (ub * 8 + static_cast<uint32_t>(2 * k + (w >> 1))) * rows16, 0));
+        r[rt].q[2] = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_raw_buffer_load_b64(o ? p11 : p10, vr[rt] * 16 + 2 * h * rows16 + w8,
+                                                        (ub * 4 + static_cast<uint32_t>(w >> 1)) * rows16, 0));
       }
     }
   };
-  if constexpr (WT == 1) {
-    // the records' zero dwords and the zero row, written once (the stash
-    // writes only the pairs)
-    for (int i = tid; i < 2 * (TOK * BSROW + BSZERO) / 8; i += 256)
-      reinterpret_cast<u32x4*>(&sBs[0][0])[i] = u32x4{0u, 0u, 0u, 0u};
-    __syncthreads();
-  }
-  fetch(0);
-  stash(0);
-  __syncthreads();
-
-  float acc[NT][8][4], accm[NT][4];
+  struct XRaw {
+    u32x4 x[NT][2];            // the token tiles' operands of lane groups 2w, 2w+1
+    f32x4 d[NT];               // d of tokens 4g .. 4g+3
+    u32x4 bs[WT == 0 ? NM : NT];  // Q4_K: bsums of tiles w, w+4, ..; Q6_K: bsums 4w .. of every tile
+    f32x4 dm[WT == 0 ? NM : 1];   // Q4_K: d of tiles w, w+4, ..
+  };
+  const __amdgpu_buffer_rsrc_t rxh = gemm_rsrc(a.xh), rxd = gemm_rsrc(a.xd), rxbs = gemm_rsrc(a.xbs);
+  const uint32_t vx = static_cast<uint32_t>(lane) * 16, vd = static_cast<uint32_t>(g) * 16;
+  const uint32_t vb = static_cast<uint32_t>(c16) * 32 + (WT == 0 ? 16u * (g & 1) : 8u * static_cast<uint32_t>(w));
+  uint32_t tb[NT], tm[NM];  // first block of each token tile
 #pragma unroll
-  for (int n = 0; n < NT; ++n) {
+  for (int n = 0; n < NT; ++n) tb[n] = static_cast<uint32_t>(min(tg * NT + n, n_tt - 1) * a.nb);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      accm[n][i] = 0.0f;
+  for (int k = 0; k < NM; ++k) tm[k] = static_cast<uint32_t>(min(tg * NT + w + 4 * k, n_tt - 1) * a.nb);
+  auto load_x = [&](XRaw& r, int n, int b) {
+    const uint32_t ub = tb[n] + static_cast<uint32_t>(b);
 #pragma unroll
-      for (int m = 0; m < 8; ++m) acc[n][m][i] = 0.0f;
+    for (int j = 0; j < 2; ++j)
+      r.x[n][j] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rxh, vx, (ub * 8 + static_cast<uint32_t>(2 * w + j)) * 1024, 0));
+    r.d[n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rxd, vd, ub * 64, 0));
+    if constexpr (WT == 1) r.bs[n] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rxbs, vb, ub * 512, 0));
+  };
+  auto load_min = [&](XRaw& r, int b) {
+    if constexpr (WT == 0) {
+#pragma unroll
+      for (int k = 0; k < NM; ++k) {
+        const uint32_t ub = tm[k] + static_cast<uint32_t>(b);
+        r.bs[k] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rxbs, vb, ub * 512, 0));
+        r.dm[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rxd, vd, ub * 64, 0));
+      }
     }
-  }
-  const h2 off1024{static_cast<_Float16>(1024.0f), static_cast<_Float16>(1024.0f)};
-  const h2 q4c16{static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
-  const h2 q4cm64{static_cast<_Float16>(-64.0f), static_cast<_Float16>(-64.0f)};
-  const h2 q4cm1024{static_cast<_Float16>(-1024.0f), static_cast<_Float16>(-1024.0f)};
+  };
+
+  f32x4 acc[RT][2][NT], accm[RT][NM];
   const f32x4 zero4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[rt][0][n] = acc[rt][1][n] = zero4;
+#pragma unroll
+    for (int k = 0; k < NM; ++k) accm[rt][k] = zero4;
+  }
+  // Q4_K, per lane: the scale bytes of sub-blocks 2g and 2g+1 as ((s0 >> sh4) &
+  // m4a) | (s2 & m4b), the min bytes of K-half g (0, 1; none for 2, 3)
+  // alike, so that no lane branches
+  const uint32_t sh4 = g < 2 ? 0u : 2u, m4a = g < 2 ? 0x3f3f3f3fu : 0x30303030u, m4b = g < 2 ? 0u : 0x0f0f0f0fu;
+  const uint32_t shm = g == 1 ? 2u : 0u, mma = g == 0 ? 0x3f3f3f3fu : g == 1 ? 0x30303030u : 0u,
+                 mmb = g == 1 ? 0x0f0f0f0fu : 0u;
+  const uint32_t sel4a = 0x04000400u | (0x00010001u * 2u * (g & 1)), sel4b = sel4a + 0x00010001u;
+  const uint32_t mac = g == 0 ? 0xffffffffu : 0u;  // Q6_K's offset pairs sit in K-half 0
   // Q6_K, per lane (K-half g: code fields at bit 4*(g&1) of each byte, and
   // the high bits' second field 2 above): field masks and the constants of
-  // the scale builds (f = 2^-p for a field at bit p)
-  struct Q6Consts {
-    uint32_t ml, ma0, ma1;
-    h2 sl1, sl2, ol1, ol2, sa1, sa2, oa1, oa2, c1, c2;
-  };
-  const Q6Consts q6c = [&] {
-    const bool odd = (g & 1) != 0;
-    const float fl = odd ? 0.0625f : 1.0f, fa = odd ? 0.015625f : 0.25f;
-    auto hs = [](float v) {
-      const _Float16 h = static_cast<_Float16>(v);
-      return h2{h, h};
-    };
-    return Q6Consts{odd ? 0xf0f0f0f0u : 0x0f0f0f0fu, odd ? 0x30303030u : 0x03030303u, odd ? 0xc0c0c0c0u : 0x0c0c0c0cu,
-                    hs(fl * 0.015625f), hs(-18.0f * fl), hs(-16.0f * fl), hs(18432.0f * fl),
-                    hs(fa * 0.015625f), hs(-18.0f * fa), hs(-16.0f * fa), hs(18432.0f * fa),
-                    hs(-0.03125f), hs(36.0f)};
-  }();
+  // the scale builds (f = 2^-p for a field at bit p; u = sc + 128):
+  // sc*f/64 = (1024 + u)*f/64 - 18*f, -16*sc*f = (1024 + u)*(-16*f) + 18432*f
+  const bool odd = (g & 1) != 0;
+  const float fl = odd ? 0.0625f : 1.0f, fa = odd ? 0.015625f : 0.25f;
+  const uint32_t ml = odd ? 0xf0f0f0f0u : 0x0f0f0f0fu, ma0 = odd ? 0x30303030u : 0x03030303u,
+                 ma1 = odd ? 0xc0c0c0c0u : 0x0c0c0c0cu;
+  const h2 sl1 = splat2(fl * 0.015625f), sl2 = splat2(-18.0f * fl), ol1 = splat2(-16.0f * fl), ol2 = splat2(18432.0f * fl);
+  const h2 sa1 = splat2(fa * 0.015625f), sa2 = splat2(-18.0f * fa), oa1 = splat2(-16.0f * fa), oa2 = splat2(18432.0f * fa);
+  const uint32_t k0 = static_cast<uint32_t>(w >> 1), k1 = 2 + k0;  // the lane groups' sub-block scales
+  const uint32_t selk0 = 0x04000400u | (k0 << 16) | k0, selk1 = 0x04000400u | (k1 << 16) | k1;
 
-  // The weight bytes a block's A operands and row scales are built from,
-  // loaded one block ahead like the activations (loaded in their own block,
-  // they would hold every block's MFMAs for a full memory round trip).
-  // Q4_K: hdr = the A row's d/dmin/scales, q[0..1] = its chunk planes 2g and
-  // 2g+1; Q6_K: hdr = its scales, q[0..3] = ql planes 4h.., q[4..5] = qh
-  // planes 2h..; dr[i] = d (and Q4_K's dmin) of D row 4g+i.
-  // (Q4_K's hdr is the 12 scale bytes only: a dword of a vector load left
-  // unused is a register the compiler reuses, and reusing it waits for every
-  // load in flight)
-  struct WRaw {
-    typename std::conditional<WT == 0, u32x3, u32x4>::type hdr;
-    u32x4 q[WT == 0 ? 2 : 6];
-    uint32_t dr[4];
-  };
-  const __amdgpu_buffer_rsrc_t rw0 = gemm_rsrc(W.p0), rw1 = gemm_rsrc(W.p1), rw2 = gemm_rsrc(W.p2),
-                               rw3 = gemm_rsrc(W.p3);
-  const uint32_t rows16 = static_cast<uint32_t>(rows) * 16;
-  uint32_t vo_dr[4];
+  // One block: the weight operands of every row tile are built, then each
+  // token tile's MFMAs and chain steps run for all of them.  Loads of block b +
+  // PF are issued as the registers they go to are read out.
+  auto block = [&](WRaw (&r)[RT], XRaw& x, int b) {
+    const int bn = min(b + PF, a.nb - 1);
+    h8 Bl[RT][2], Bh[RT][2], Bc[RT][2];
+    float dw[RT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    vo_dr[i] = static_cast<uint32_t>(min(r0 + 4 * g + i, rows - 1)) * (WT == 0 ? 16u : 2u);
-  const uint32_t vo_ra = static_cast<uint32_t>(ra) * 16;
-  auto load_w = [&](WRaw& w, int b) {
-    const uint32_t ub = static_cast<uint32_t>(b);
-    if constexpr (WT == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w.dr[i] = __builtin_amdgcn_raw_buffer_load_b32(rw1, vo_dr[i], ub * rows16, 0);
-      w.hdr = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(rw1, vo_ra + 4, ub * rows16, 0));
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        w.q[j] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw0, vo_ra + (2 * g + j) * rows16, ub * 8 * rows16, 0));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        w.dr[i] = __builtin_amdgcn_raw_buffer_load_b16(rw3, vo_dr[i], ub * static_cast<uint32_t>(rows) * 2, 0);
-      const int h = g >> 1;
-      w.hdr = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw2, vo_ra, ub * rows16, 0));
-#pragma unroll
-      for (int cc = 0; cc < 4; ++cc)
-        w.q[cc] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw0, vo_ra + (4 * h + cc) * rows16, ub * 8 * rows16, 0));
-#pragma unroll
-      for (int cc = 0; cc < 2; ++cc)
-        w.q[4 + cc] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw1, vo_ra + (2 * h + cc) * rows16, ub * 4 * rows16, 0));
-    }
-  };
-  // One block: the weight bytes of block b+1 (into nxt) and its activations
-  // are loaded while block b's MFMAs run; cur and nxt trade places each
-  // block, so no copy waits for loads in flight.
-  auto block = [&](int b, const WRaw& wc, WRaw& wn) {
-    const int buf = b & 1;
-    // in flight during this block's MFMAs; issued unconditionally (the last
-    // block loads itself again, unused), so the wait for wc's loads counts
-    // the same number of younger loads on every path and leaves these in
-    // flight
-    const int bn = min(b + 1, a.nb - 1);
-    fetch(bn);
-    load_w(wn, bn);
-    if (live) {
-    // d (and dmin) of the four D rows of this lane
-    float dw[4], dmw[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int rt = 0; rt < RT; ++rt) {
       if constexpr (WT == 0) {
-        dw[i] = fp16_to_fp32(static_cast<uint16_t>(wc.dr[i] & 0xffffu));
-        dmw[i] = fp16_to_fp32(static_cast<uint16_t>(wc.dr[i] >> 16));
+        dw[rt] = fp16_to_fp32(static_cast<uint16_t>(r[rt].hdr.x & 0xffffu));
+        const uint32_t s0 = r[rt].hdr.y, s1 = r[rt].hdr.z, s2 = r[rt].hdr.w;
+        // sc[2g] over 64 (low nibbles) and sc[2g+1] over 1024 (high nibbles,
+        // read in place as 16*code), and the offsets -1024*s
+        const uint32_t sw = ((s0 >> sh4) & m4a) | (s2 & m4b);
+        const h2 ha = byte_pair(sw, sel4a), hb = byte_pair(sw, sel4b);
+        const h2 sa = __builtin_elementwise_fma(ha, splat2(0.015625f), splat2(-16.0f));
+        const h2 sb = __builtin_elementwise_fma(hb, splat2(0.0009765625f), splat2(-1.0f));
+        const h2 ma = sa * splat2(-1024.0f), mb = sb * splat2(-1024.0f);
+        const uint32_t q0 = r[rt].q[0].x, q1 = r[rt].q[0].y;
+        Bl[rt][0] = w_operand(q0 & 0x0f0f0f0fu, q0 & 0xf0f0f0f0u, sa, sb, ma, mb);
+        Bl[rt][1] = w_operand(q1 & 0x0f0f0f0fu, q1 & 0xf0f0f0f0u, sa, sb, ma, mb);
+        // the min chain of token tiles w, w+4, ..: k = 8g + j < 16 -> mn[k/2]
+        const float dmw = fp16_to_fp32(static_cast<uint16_t>(r[rt].hdr.x >> 16));
+        const uint32_t mw = ((s1 >> shm) & mma) | ((s2 >> 4) & mmb);  // 0 for K-halves 2, 3
+        const h2 o1024 = splat2(1024.0f);
+        const u32x4 mr{h2bits(byte_pair(mw, 0x04000400u) - o1024), h2bits(byte_pair(mw, 0x04010401u) - o1024),
+                       h2bits(byte_pair(mw, 0x04020402u) - o1024), h2bits(byte_pair(mw, 0x04030403u) - o1024)};
+        const h8 BM = __builtin_bit_cast(h8, mr);
+#pragma unroll
+        for (int k = 0; k < NM; ++k) {
+          const f32x4 DM = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, x.bs[k]), BM, zero4, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) accm[rt][k][i] = __builtin_fmaf(-(x.dm[k][i] * dmw), DM[i], accm[rt][k][i]);
+        }
       } else {
-        dw[i] = fp16_to_fp32(static_cast<uint16_t>(wc.dr[i]));
-        dmw[i] = 0.0f;
+        dw[rt] = fp16_to_fp32(static_cast<uint16_t>(r[rt].hdr.z));
+        const uint32_t su = r[rt].hdr.x ^ 0x80808080u, sc = r[rt].hdr.y ^ 0x80808080u;
+        const h2 ha = byte_pair(su, selk0), hb = byte_pair(su, selk1);
+        const h2 sLa = __builtin_elementwise_fma(ha, sl1, sl2), oLa = __builtin_elementwise_fma(ha, ol1, ol2);
+        const h2 sLb = __builtin_elementwise_fma(hb, sl1, sl2), oLb = __builtin_elementwise_fma(hb, ol1, ol2);
+        const h2 sAb = __builtin_elementwise_fma(hb, sa1, sa2), oAb = __builtin_elementwise_fma(hb, oa1, oa2);
+        // (qh's first field is at the bit of the low codes' field: its factor)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const uint32_t la = j ? r[rt].q[0].y : r[rt].q[0].x, lb = j ? r[rt].q[1].y : r[rt].q[1].x;
+          const uint32_t hq = j ? r[rt].q[2].y : r[rt].q[2].x;
+          Bl[rt][j] = w_operand(la & ml, lb & ml, sLa, sLb, oLa, oLb);
+          Bh[rt][j] = w_operand(hq & ma0, hq & ma1, sLa, sAb, oLa, oAb);
+          // the offset pair -2*sc of sub-blocks 2m, 2m+1 = (1024 + u)*(-2) +
+          // 2304, against the bsums 2m, 2m+1 that K-half 0 holds at dword j
+          const h2 hp = byte_pair(sc, 0x04000400u | ((2u * j + 1) << 16) | (2u * j));
+          const uint32_t ac = h2bits(__builtin_elementwise_fma(hp, splat2(-2.0f), splat2(2304.0f))) & mac;
+          Bc[rt][j] = __builtin_bit_cast(h8, j ? u32x4{0u, ac, 0u, 0u} : u32x4{ac, 0u, 0u, 0u});
+        }
       }
     }
-    // Lane groups in order; each one's A operand is built from the weight
-    // bytes just before its MFMAs (one per token tile, the operand then
-    // dropped), so the build of the next overlaps them.
-    float ds[NT][4], xdv[NT];
+    load_w(r, bn);
+    load_min(x, bn);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
-      xdv[n] = sXd[buf][16 * n + c16];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ds[n][i] = WT == 0 ? xdv[n] * dw[i] : (xdv[n] * dw[i]) * 64.0f;
+      for (int rt = 0; rt < RT; ++rt) {
+        f32x4 S[2], T[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const h8 A = __builtin_bit_cast(h8, x.x[n][j]);
+          S[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, Bl[rt][j], zero4, 0, 0, 0);
+          if constexpr (WT == 1) {
+            T[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, x.bs[n]), Bc[rt][j], zero4, 0, 0, 0);
+            T[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, Bh[rt][j], T[j], 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float ds = x.d[n][i] * dw[rt];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float v = WT == 0 ? S[j][i] : __builtin_fmaf(16.0f, T[j][i], S[j][i]);
+            acc[rt][j][n][i] = __builtin_fmaf(ds, v, acc[rt][j][n][i]);
+          }
+        }
+      }
+      load_x(x, n, bn);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // the B operand of lane group m for token tile n is quad 8g + m of the
-    // token's row (at slot (8g + m) ^ sw(g))
-    auto bq = [&](int n, int m) {
-      return __builtin_bit_cast(h8, reinterpret_cast<const u32x4*>(&sB[buf][(16 * n + c16) * BROW])[(8 * g + m) ^ ((g ^ (g >> 1)) & 1)]);
-    };
-    if constexpr (WT == 0) {
-      const uint32_t s0 = wc.hdr.x, s1 = wc.hdr.y, s2 = wc.hdr.z;
-      const uint32_t sc_lo = s0 & 0x3f3f3f3fu;
-      const uint32_t sc_hi = (s2 & 0x0f0f0f0fu) | ((s0 >> 2) & 0x30303030u);
-      const uint32_t mn_lo = s1 & 0x3f3f3f3fu;
-      const uint32_t mn_hi = ((s2 >> 4) & 0x0f0f0f0fu) | ((s1 >> 2) & 0x30303030u);
-      // sc[2g] (low nibbles) and sc[2g+1]/16 (high nibbles, read in place as
-      // 16*code), from fp16 (1024 + sc) by byte permute; the offsets -1024*s
-      // (exact: sc <= 63)
-      const uint32_t sw = g < 2 ? sc_lo : sc_hi;
-      const uint32_t bs = 2 * (g & 1);
-      const h2 ha = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, sw, 0x04000400u | (bs << 16) | bs));
-      const h2 hb = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, sw, 0x04000400u | ((bs + 1) << 16) | (bs + 1)));
-      const h2 sa = ha - off1024, sb = __builtin_elementwise_fma(hb, q4c16, q4cm64);
-      const h2 ma = sa * q4cm1024, mb = sb * q4cm1024;
-      const u32x4 q0 = wc.q[0], q1 = wc.q[1];
-      const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-      // two lane groups at a time: their 2*NT MFMAs are independent and
-      // issue back to back before the first chain step reads a result; the
-      // next pair's B operands are read from LDS while this pair's run
-      h8 Bc[2][NT];
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        Bc[0][n] = bq(n, 0);
-        Bc[1][n] = bq(n, 1);
-      }
-#pragma unroll
-      for (int m = 0; m < 8; m += 2) {
-        h8 Bn[2][NT];
-        if (m + 2 < 8) {
-#pragma unroll
-          for (int n = 0; n < NT; ++n) {
-            Bn[0][n] = bq(n, m + 2);
-            Bn[1][n] = bq(n, m + 3);
-          }
-        }
-        const h8 A0 = a_operand_fma(qw[m] & 0x0f0f0f0fu, qw[m] & 0xf0f0f0f0u, sa, sb, ma, mb);
-        const h8 A1 = a_operand_fma(qw[m + 1] & 0x0f0f0f0fu, qw[m + 1] & 0xf0f0f0f0u, sa, sb, ma, mb);
-        f32x4 D0[NT], D1[NT];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-          D0[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, Bc[0][n], zero4, 0, 0, 0);
-          D1[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, Bc[1][n], zero4, 0, 0, 0);
-        }
-        if (m + 2 < 8) {
-#pragma unroll
-          for (int n = 0; n < NT; ++n) {
-            Bc[0][n] = Bn[0][n];
-            Bc[1][n] = Bn[1][n];
-          }
-        }
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            acc[n][m][i] = __builtin_fmaf(ds[n][i], D0[n][i], acc[n][m][i]);
-            acc[n][m + 1][i] = __builtin_fmaf(ds[n][i], D1[n][i], acc[n][m + 1][i]);
-          }
-        }
-      }
-      // min operand: k = 8g + j < 16 -> mn[k/2]
-      const uint32_t mw = (g & 1) ? mn_hi : mn_lo;
-      const u32x4 mr{h2bits(byte_pair_h(mw, 0x04000400u, off1024)), h2bits(byte_pair_h(mw, 0x04010401u, off1024)),
-                     h2bits(byte_pair_h(mw, 0x04020402u, off1024)), h2bits(byte_pair_h(mw, 0x04030403u, off1024))};
-      const h8 AM = g < 2 ? __builtin_bit_cast(h8, mr) : h8{};
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const h8 BM = *reinterpret_cast<const h8*>(&sBs[buf][(16 * n + c16) * BSROW + 8 * (g & 1)]);
-        const f32x4 DM = __builtin_amdgcn_mfma_f32_16x16x32_f16(AM, BM, zero4, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) accm[n][i] = __builtin_fmaf(-(xdv[n] * dmw[i]), DM[i], accm[n][i]);
-      }
-    } else {
-      // The 16 scales as unsigned bytes u = sc + 128; fp16 (1024 + u) from a
-      // byte permute, then one packed fma gives sc*f/64 = (1024 + u)*f/64 -
-      // 18*f or -16*sc*f = (1024 + u)*(-16*f) + 18432*f, exactly (f a power of
-      // two).  The lane's code fields are masked in place (not shifted): a
-      // field at bit p of its byte reads as code*2^p, and its scale carries
-      // f = 2^-p, so every A entry is still code*sc/64.
-      const u32x4 scr = wc.hdr;
-      const uint32_t su[4] = {scr.x ^ 0x80808080u, scr.y ^ 0x80808080u, scr.z ^ 0x80808080u, scr.w ^ 0x80808080u};
-      const uint32_t scw = g == 0 ? su[0] : g == 1 ? su[1] : g == 2 ? su[2] : su[3];  // scales 4g .. 4g+3
-      h2 sL[4], oL[4], sA[2], oA[2];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const h2 hb = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, scw, 0x04000400u | (k << 16) | k));
-        sL[k] = __builtin_elementwise_fma(hb, q6c.sl1, q6c.sl2);
-        oL[k] = __builtin_elementwise_fma(hb, q6c.ol1, q6c.ol2);
-        if (k >= 2) {
-          sA[k - 2] = __builtin_elementwise_fma(hb, q6c.sa1, q6c.sa2);
-          oA[k - 2] = __builtin_elementwise_fma(hb, q6c.oa1, q6c.oa2);
-        }
-      }
-      uint32_t lw[16], hw[8];
-#pragma unroll
-      for (int cc = 0; cc < 4; ++cc) {
-        const u32x4 v = wc.q[cc];
-        lw[4 * cc] = v.x;
-        lw[4 * cc + 1] = v.y;
-        lw[4 * cc + 2] = v.z;
-        lw[4 * cc + 3] = v.w;
-      }
-#pragma unroll
-      for (int cc = 0; cc < 2; ++cc) {
-        const u32x4 v = wc.q[4 + cc];
-        hw[4 * cc] = v.x;
-        hw[4 * cc + 1] = v.y;
-        hw[4 * cc + 2] = v.z;
-        hw[4 * cc + 3] = v.w;
-      }
-      // one lane group's operands; two lane groups' MFMAs are issued before
-      // either chain reads a result
-      auto q6_ops = [&](int m, h8& Al, h8& Ah, uint32_t& AC) {
-        const int ka = m >> 2, kb = 2 + (m >> 2);
-        Al = a_operand_fma(lw[m] & q6c.ml, lw[8 + m] & q6c.ml, sL[ka], sL[kb], oL[ka], oL[kb]);
-        Ah = a_operand_fma(hw[m] & q6c.ma0, hw[m] & q6c.ma1, sL[ka], sA[kb - 2], oL[ka], oA[kb - 2]);
-        // the offset operand's first K pair: -2*sc[2m]/64, -2*sc[2m+1]/64 of
-        // this lane's row (-sc/32 = (1024 + u)*(-1/32) + 36)
-        const uint32_t sel = 0x04000400u | ((2 * (m & 1) + 1) << 16) | (2 * (m & 1));
-        const h2 hp = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, su[m >> 1], sel));
-        AC = h2bits(__builtin_elementwise_fma(hp, q6c.c1, q6c.c2));
-      };
-      // S + 16*T for lane group m and token tile n: S = sc*ql*x, T = sc*qh*x - 2C
-      // (each divided by 64, exactly)
-      // the B operand and the bsums pair of lane group m, token tile n
-      struct BOp {
-        h8 B;
-        h8 BC;  // record m of the token (lanes 0..15), the zero row (the others)
-      };
-      auto b_op = [&](int m, int n) {
-        const int row = g == 0 ? (16 * n + c16) * BSROW : TOK * BSROW;
-        return BOp{bq(n, m), *reinterpret_cast<const h8*>(&sBs[buf][row + m * 8])};
-      };
-      // The offset operand is Al with its first dword replaced by the pair
-      // (formed after the S MFMAs have read Al): its other K entries meet
-      // zeros of BC, and lanes 16..63 read an all-zero BC, so NC is the
-      // offset alone.
-      auto q6_mfma = [&](const BOp& o, const h8& Al, const h8& Ah, uint32_t AC, f32x4& S, f32x4& T) {
-        S = __builtin_amdgcn_mfma_f32_16x16x32_f16(Al, o.B, zero4, 0, 0, 0);
-        const u32x4 al = __builtin_bit_cast(u32x4, Al);
-        const h8 A2 = __builtin_bit_cast(h8, u32x4{AC, al.y, al.z, al.w});
-        const f32x4 NC = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2, o.BC, zero4, 0, 0, 0);  // -2C
-        T = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ah, o.B, NC, 0, 0, 0);
-      };
-      // Lane groups in steps of LG: pairs with one token tile (their six
-      // MFMAs independent), one at a time with two (registers: two tiles'
-      // accumulators, sums and B operands).  The next step's B operands are
-      // read from LDS while this step's MFMAs run.
-      constexpr int LG = NT >= 2 ? 1 : 2;
-      BOp Oc[LG][NT];
-#pragma unroll
-      for (int j = 0; j < LG; ++j) {
-#pragma unroll
-        for (int n = 0; n < NT; ++n) Oc[j][n] = b_op(j, n);
-      }
-#pragma unroll
-      for (int m = 0; m < 8; m += LG) {
-        BOp On[LG][NT];
-        if (m + LG < 8) {
-#pragma unroll
-          for (int j = 0; j < LG; ++j) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) On[j][n] = b_op(m + LG + j, n);
-          }
-        }
-        h8 Al[LG], Ah[LG];
-        uint32_t AC[LG];
-#pragma unroll
-        for (int j = 0; j < LG; ++j) q6_ops(m + j, Al[j], Ah[j], AC[j]);
-        f32x4 S[LG][NT], T[LG][NT];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-#pragma unroll
-          for (int j = 0; j < LG; ++j) q6_mfma(Oc[j][n], Al[j], Ah[j], AC[j], S[j][n], T[j][n]);
-        }
-        if (m + LG < 8) {
-#pragma unroll
-          for (int j = 0; j < LG; ++j) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) Oc[j][n] = On[j][n];
-          }
-        }
-#pragma unroll
-        for (int n = 0; n < NT; ++n) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < LG; ++j)
-              acc[n][m + j][i] = __builtin_fmaf(ds[n][i], __builtin_fmaf(16.0f, T[j][n][i], S[j][n][i]), acc[n][m + j][i]);
-          }
-        }
-      }
-    }
-    }  // live
-    // block b+1 into the other buffer, whose last readers passed the previous
-    // barrier (after the last block: a copy of it, never read)
-    stash(buf ^ 1);
-    __syncthreads();
   };
-  WRaw w0, w1;
-  load_w(w0, 0);
-  // pairs of blocks with no branch inside, then the odd block
-  int b = 0;
-  for (; b + 1 < a.nb; b += 2) {
-    block(b, w0, w1);
-    block(b + 1, w1, w0);
-  }
-  if (b < a.nb) block(b, w0, w1);
 
-  float vs[NT][4];
+  WRaw wr[PF][RT];
+  XRaw xr[PF];
+  // oldest first: a wait for a load waits for every older one
 #pragma unroll
-  for (int n = 0; n < NT; ++n) {
+  for (int p = 0; p < PF; ++p) {
+    load_w(wr[p], min(p, a.nb - 1));
+    load_min(xr[p], min(p, a.nb - 1));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      vs[n][i] = ((acc[n][0][i] + acc[n][4][i]) + (acc[n][2][i] + acc[n][6][i])) +
-                 ((acc[n][1][i] + acc[n][5][i]) + (acc[n][3][i] + acc[n][7][i]));
-      if constexpr (WT == 0) vs[n][i] = vs[n][i] + accm[n][i];
-    }
+    for (int n = 0; n < NT; ++n) load_x(xr[p], n, min(p, a.nb - 1));
   }
-  if (a.swiglu) {
-    // the up waves hand their values to the gate waves of the same rows and
-    // tokens through LDS (sB is free: every read of it passed the last
-    // block's barrier)
-    float* xs = reinterpret_cast<float*>(&sB[0][0]);
-    if (second) {
+  // groups of PF blocks with no branch inside (the waits for the loads then
+  // count exactly), then the remainder
+  int b = 0;
+  for (; b + PF <= a.nb; b += PF) {
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
+    for (int p = 0; p < PF; ++p) block(wr[p], xr[p], b + p);
+  }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) xs[(((wv & 1) * NT + n) * 4 + i) * 64 + lane] = vs[n][i];
-      }
+  for (int p = 0; p < PF - 1; ++p)
+    if (b + p < a.nb) block(wr[p], xr[p], b + p);
+
+  // Row tile by row tile, the waves put their lane groups' chains together:
+  // wave w finishes token tiles w, w+4, ...
+  f32x4 gate[NM];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    if (rt) __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) s_acc[((2 * w + j) * NT + n) * 64 + lane] = acc[rt][j][n];
     }
     __syncthreads();
-    if (second) return;
+    const int r = row0(rt) + c16;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
+    for (int k = 0; k < NM; ++k) {
+      const int n = w + 4 * k;
+      if (n >= NT) break;
+      f32x4 m[8], v;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) m[j] = s_acc[(j * NT + n) * 64 + lane];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float gv = vs[n][i], uv = xs[(((wv & 1) * NT + n) * 4 + i) * 64 + lane];
-        vs[n][i] = (gv / (1.0f + exp_f32(-gv))) * uv;
+        v[i] = ((m[0][i] + m[4][i]) + (m[2][i] + m[6][i])) + ((m[1][i] + m[5][i]) + (m[3][i] + m[7][i]));
+        if constexpr (WT == 0) v[i] = v[i] + accm[rt][k][i];
       }
-    }
-  }
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    const int t = t0 + 16 * n + c16;
-    float v[4] = {vs[n][0], vs[n][1], vs[n][2], vs[n][3]};
-    if (a.rope) {
-      // rows 4g+i of the lane: pairs (0, 1) and (2, 3), apply_rope's
-      // products and sums (src/ops/ops.cpp:502-516)
-      const size_t pos = static_cast<size_t>(a.pos0 + min(t, a.n_tok - 1));
-#pragma unroll
-      for (int i = 0; i < 4; i += 2) {
-        const int d = (r0 + 4 * g + i) % a.rope_hd;
-        const float2 cs = a.rope[pos * (a.rope_hd / 2) + (d >> 1)];
-        const float e = v[i], o = v[i + 1];
-        v[i] = e * cs.x - o * cs.y;
-        v[i + 1] = e * cs.y + o * cs.x;
-      }
-    }
-    // the lane's four rows are consecutive: one 16-byte access where all
-    // four exist and the address is aligned, else one by one
-    const int r4 = r0 + 4 * g;
-    float* o = out + static_cast<size_t>(min(t, a.n_tok - 1)) * ld_out + r4;
-    if (t < a.n_tok) {
-      if (r4 + 3 < rows && (reinterpret_cast<uintptr_t>(o) & 15) == 0) {
-        f32x4 w{v[0], v[1], v[2], v[3]};
-        if (a.add) {
-          const f32x4 p = *reinterpret_cast<const f32x4*>(o);
-          w = f32x4{p.x + v[0], p.y + v[1], p.z + v[2], p.w + v[3]};
+      if (a.swiglu) {
+        if ((rt & 1) == 0) {
+          gate[k] = v;
+          continue;
         }
-        *reinterpret_cast<f32x4*>(o) = w;
-      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = (gate[k][i] / (1.0f + exp_f32(-gate[k][i]))) * v[i];
+      }
+      const int t4 = 16 * (tg * NT + n) + 4 * g;  // the lane's first token
+      if (a.rope) {
+        // rows (2i, 2i+1) of a pair are neighbouring lanes; apply_rope's
+        // products and sums (src/ops/ops.cpp:502-516)
+        const int d = (r % a.rope_hd) >> 1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const size_t pos = static_cast<size_t>(a.pos0 + min(t4 + i, a.n_tok - 1));
+          const float2 cs = a.rope[pos * (a.rope_hd / 2) + d];
+          const float o = dpp_f<DPP_XOR1>(v[i]);
+          v[i] = (c16 & 1) ? o * cs.y + v[i] * cs.x : v[i] * cs.x - o * cs.y;
+        }
+      }
+      if (r < rows) {
+        float* o = (second ? a.out2 : a.out) + r;
+        const size_t ld = second ? a.ld_out2 : a.ld_out;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (r4 + i < rows) o[i] = a.add ? o[i] + v[i] : v[i];
+          if (t4 + i < a.n_tok) o[(t4 + i) * ld] = a.add ? o[(t4 + i) * ld] + v[i] : v[i];
       }
     }
   }
@@ -792,9 +616,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, 8
 __global__ void __launch_bounds__(256) k_quant_batch_attn(const float* __restrict__ part_o,
                                                           const float2* __restrict__ part_mz, size_t tok_stride_o,
                                                           size_t tok_stride_mz, int pos0, int dim, int hd,
-                                                          int max_chunks, _Float16* __restrict__ xh,
+                                                          int max_chunks, int n_tok, _Float16* __restrict__ xh,
                                                           float* __restrict__ xd, _Float16* __restrict__ xbs) {
-  const int t = blockIdx.x;
+  const int t = quant_token(blockIdx.x);
+  if (t >= n_tok) return;  // uniform, before any barrier
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nch = (pos0 + t) / ATTN_CHUNK + 1;
   const int nb = dim / QK_K;
@@ -845,12 +670,7 @@ __global__ void __launch_bounds__(256) k_quant_batch_attn(const float* __restric
     float dq;
     int gsum;
     quant_block_wave(v, false, packed, dq, gsum);
-    _Float16* out = xh + static_cast<size_t>(t) * dim + i0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      out[k] = static_cast<_Float16>(static_cast<float>(static_cast<int8_t>((packed >> (8 * k)) & 0xffu)));
-    if ((lane & 3) == 0) xbs[(static_cast<size_t>(t) * nb + b) * 16 + (lane >> 2)] = static_cast<_Float16>(gsum);
-    if (lane == 0) xd[static_cast<size_t>(t) * nb + b] = dq;
+    store_codes(t, nb, b, lane, packed, dq, gsum, xh, xd, xbs);
   }
 }
 
@@ -868,14 +688,14 @@ hipError_t launch_quant_batch(const float* x, const float* u, int ld_x, const fl
   if (n_valid < 1 || n_valid > dim || n_valid > ld_x) return hipErrorInvalidValue;
   const bool up_front = ld_x % 4 == 0 && n_valid % 4 == 0;
   if (up_front && nb <= 12)
-    hipLaunchKernelGGL(k_quant_batch_r<3>, dim3(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid, mode,
-                       q.xh, q.xd, q.xbs);
+    hipLaunchKernelGGL(k_quant_batch_r<3>, quant_grid(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid,
+                       mode, n_tok, q.xh, q.xd, q.xbs);
   else if (up_front && nb <= 24)
-    hipLaunchKernelGGL(k_quant_batch_r<6>, dim3(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid, mode,
-                       q.xh, q.xd, q.xbs);
+    hipLaunchKernelGGL(k_quant_batch_r<6>, quant_grid(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid,
+                       mode, n_tok, q.xh, q.xd, q.xbs);
   else
-    hipLaunchKernelGGL(k_quant_batch, dim3(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid, mode,
-                       q.xh, q.xd, q.xbs);
+    hipLaunchKernelGGL(k_quant_batch, quant_grid(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid,
+                       mode, n_tok, q.xh, q.xd, q.xbs);
   return hipGetLastError();
 }
 
@@ -888,48 +708,45 @@ hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const Qu
                            bool add, hipStream_t s, const WView* w2, int rows2, float* out2, int ld_out2,
                            const GemmRope* rope, bool swiglu) {
   if (w.type != MCPM_TYPE_Q4_K && w.type != MCPM_TYPE_Q6_K) return hipErrorInvalidValue;
-  if (rows2 > 0 && (!w2 || w2->type != w.type || rows % 64 || (!swiglu && !out2))) return hipErrorInvalidValue;
-  if (swiglu && (rows2 != rows || rows % 32 || rope || add)) return hipErrorInvalidValue;
-  // a rotated pair (rows 2i, 2i+1) stays in one head and one lane: head_dim
-  // even, every matrix's rows a multiple of it
+  if (rows < 1 || nb < 1 || n_tok < 1) return hipErrorInvalidValue;
+  if (rows2 > 0 && (!w2 || w2->type != w.type || (!swiglu && !out2))) return hipErrorInvalidValue;
+  if (swiglu && (rows2 != rows || rope || add)) return hipErrorInvalidValue;
+  // a rotated pair (rows 2i, 2i+1) stays in one head and one row tile:
+  // head_dim even, every matrix's rows a multiple of it
   if (rope && (!rope->table || rope->head_dim <= 0 || rope->head_dim % 2 || rows % rope->head_dim ||
                (rows2 > 0 && rows2 % rope->head_dim)))
     return hipErrorInvalidValue;
   GemmArgs a{w, rows, nb, n_tok, q.xh, q.xd, q.xbs, out, ld_out, add ? 1 : 0, rows2 > 0 ? *w2 : WView{},
              std::max(rows2, 0), out2, ld_out2, rope ? rope->table : nullptr, rope ? rope->head_dim : 0,
              rope ? rope->pos0 : 0, swiglu ? 1 : 0};
-  rows += std::max(rows2, 0);
-  // token tiles per wave and waves per SIMD (MCPM_PREFILL_NT=1|2|4 and
-  // MCPM_PREFILL_OCC=1|2 override, tuning aids; "a,b" sets Q4_K a, Q6_K b)
-  struct Pair {
-    int q4 = 0, q6 = 0;
-  };
-  auto env_pair = [](const char* name) {
-    Pair p;
-    if (const char* v = std::getenv(name)) {
-      const int n = std::sscanf(v, "%d,%d", &p.q4, &p.q6);
-      if (n == 1) p.q6 = p.q4;
-    }
-    return p;
-  };
-  static const Pair nt_env = env_pair("MCPM_PREFILL_NT"), occ_env = env_pair("MCPM_PREFILL_OCC");
   const bool q4 = w.type == MCPM_TYPE_Q4_K;
-  const int nt_e = q4 ? nt_env.q4 : nt_env.q6, occ_e = q4 ? occ_env.q4 : occ_env.q6;
-  // Defaults: two waves per SIMD (registers held to 256 so a second wave hides
-  // the first's load latency); 32 tokens per wave for Q4_K, 16 for Q6_K, whose
-  // four MFMA operand sets need the room.
-  const int NT = nt_e == 1 || nt_e == 2 || nt_e == 4 ? nt_e : (q4 ? 2 : 1);
-  const int OCC = occ_e == 1 ? 1 : 2;
-  // one work group per 64 rows (four 16-row tiles) x 16*NT tokens: per XCD,
-  // q row groups x token tiles and a share of the other r (see k_gemm_q8k)
-  const int n_rg = (rows + 63) / 64, n_tg = (n_tok + 16 * NT - 1) / (16 * NT);
+  // Token tiles per work group: building a block's weight operands costs about
+  // two tiles' chains, so NT token tiles per group cost ceil(tiles / NT) * (2 +
+  // NT); the fewest, up to 4 (the registers of two waves per SIMD).  Two row
+  // tiles per work group share each activation operand where that still leaves
+  // a work group per CU, else one (2304 rows, 76 tokens: 144 work groups of
+  // two, 5.53 ms a prompt, 5.20 with one); gate and up always pair.
+  const int tiles = (n_tok + 15) / 16;
+  int NT = 1;
+  for (int n = 2; n <= 4; ++n)
+    if ((tiles + n - 1) / n * (2 + n) < (tiles + NT - 1) / NT * (2 + NT)) NT = n;
+  const int n_tg = (tiles + NT - 1) / NT;
+  auto groups = [&](int rpg) { return (rows + rpg - 1) / rpg + (swiglu ? 0 : (std::max(rows2, 0) + rpg - 1) / rpg); };
+  const int RT = swiglu || groups(32) * n_tg >= 256 ? 2 : 1;
+  const int n_rg = groups(swiglu ? 16 : 16 * RT);
   const dim3 grid(8 * ((n_rg / 8) * n_tg + ((n_rg % 8) * n_tg + 7) / 8));
-#define MCPM_GEMM(N, O) \
-  if (NT == N && OCC == O) { \
-    if (q4) launch_kernel(k_gemm_q8k<0, N, O>, grid, dim3(256), 0, s, a); \
-    else launch_kernel(k_gemm_q8k<1, N, O>, grid, dim3(256), 0, s, a); \
+  // Blocks in flight: two where a block's work is short (few tokens, weights
+  // from HBM: 2304 x 5888 Q6_K, 12 tokens, 18.9 us with one, 12.8 with two,
+  // 12.6 with four), one where the other wave of the SIMD fills the wait and
+  // the registers are better spent (1023 tokens: 21.4 ms a prompt with two
+  // blocks of weights, 20.5 with one).
+#define MCPM_GEMM(R, N, P) \
+  if (RT == R && NT == N) { \
+    if (q4) launch_kernel(k_gemm_q8k<0, R, N, P>, grid, dim3(256), 0, s, a); \
+    else launch_kernel(k_gemm_q8k<1, R, N, P>, grid, dim3(256), 0, s, a); \
   }
-  MCPM_GEMM(1, 1) MCPM_GEMM(1, 2) MCPM_GEMM(2, 1) MCPM_GEMM(2, 2) MCPM_GEMM(4, 1) MCPM_GEMM(4, 2)
+  MCPM_GEMM(1, 1, 2) MCPM_GEMM(1, 2, 2) MCPM_GEMM(1, 3, 2) MCPM_GEMM(1, 4, 2)
+  MCPM_GEMM(2, 1, 2) MCPM_GEMM(2, 2, 2) MCPM_GEMM(2, 3, 1) MCPM_GEMM(2, 4, 1)
 #undef MCPM_GEMM
   return hipGetLastError();
 }
@@ -938,8 +755,8 @@ hipError_t launch_quant_batch_attn(const AttnPart& part, size_t tok_stride_o, si
                                   int n_tok, int n_heads, int head_dim, int max_chunks, QuantBatch q, hipStream_t s) {
   const int dim = n_heads * head_dim;
   if (dim % QK_K || head_dim % 4) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_quant_batch_attn, dim3(n_tok), dim3(256), 0, s, part.o, part.mz, tok_stride_o, tok_stride_mz,
-                     pos0, dim, head_dim, max_chunks, q.xh, q.xd, q.xbs);
+  hipLaunchKernelGGL(k_quant_batch_attn, quant_grid(n_tok), dim3(256), 0, s, part.o, part.mz, tok_stride_o, tok_stride_mz,
+                     pos0, dim, head_dim, max_chunks, n_tok, q.xh, q.xd, q.xbs);
   return hipGetLastError();
 }
 
