@@ -183,133 +183,6 @@ hipError_t launch_kv_append(const float* k, const float* v, float* kc, float* vc
 }
 
 
-// NT consecutive tokens (token k with context Tk[k], k < NT; every Tk[k] >
-// c*ATTN_CHUNK) on one chunk: each token's sums are attn_token_chunk's, in
-// the same order, and the tokens' chains run side by side, so each K and V
-// value read from LDS serves NT tokens.  Token k's queries at sQ + k*QSZ, its
-// softmax terms at sE + k*ESZ, its (m_c, z_c) at mz[k*ATTN_MAX_GROUP + hh], its
-// outputs in o[k].
-// GM: the most query heads per kv head that sQ and sE hold.  SWZ: K rows
-// unpadded, 64 floats apart, float4 c4 of row j at (c4 ^ (j % 16)) (distinct
-// banks across 16 rows read together, as the padding gives).  (m_c, z_c) go
-// to put_mz(k, hh, value) from lane 0 of the head's wave.
-template <int HDM, int OPT, int NT, bool WL, int GM, bool SWZ, class PutMZ>
-__device__ __forceinline__ void attn_tokens_chunk(const float* sK, const float* sV, const float* sQ, float* sE,
-                                                  PutMZ put_mz, int c, const int (&Tk)[NT], int group, int hd, int gh,
-                                                  float scale, float (&o)[NT][OPT]) {
-  constexpr int KS = SWZ ? HDM : HDM + 4;
-  constexpr int QSZ = GM * HDM, ESZ = GM * ATTN_CHUNK;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // float offset of dimension i (a multiple of 4) in this lane's K row
-  auto kof = [&](int i) { return SWZ ? (((i >> 2) ^ (lane & 15)) << 2) : i; };
-  for (int hh = wave; hh < group; hh += 4) {
-    const float* kt = &sK[lane * KS];
-    const float* qh = sQ + hh * HDM;
-    float dot[NT];
-#pragma unroll
-    for (int k = 0; k < NT; ++k) dot[k] = 0.0f;
-    // the next 4 dimensions' K and q are read while this step's fmas run
-    // (the last step reads itself again)
-    f32x4 kc4 = *reinterpret_cast<const f32x4*>(kt + kof(0)), qc4[NT];
-#pragma unroll
-    for (int k = 0; k < NT; ++k) qc4[k] = *reinterpret_cast<const f32x4*>(qh + k * QSZ);
-#pragma unroll 2
-    for (int i = 0; i < hd; i += 4) {
-      const int in = min(i + 4, hd - 4);
-      const f32x4 kn4 = *reinterpret_cast<const f32x4*>(kt + kof(in));
-      f32x4 qn4[NT];
-#pragma unroll
-      for (int k = 0; k < NT; ++k) qn4[k] = *reinterpret_cast<const f32x4*>(qh + k * QSZ + in);
-#pragma unroll
-      for (int k = 0; k < NT; ++k) {
-        dot[k] = __builtin_fmaf(qc4[k].x, kc4.x, dot[k]);
-        dot[k] = __builtin_fmaf(qc4[k].y, kc4.y, dot[k]);
-        dot[k] = __builtin_fmaf(qc4[k].z, kc4.z, dot[k]);
-        dot[k] = __builtin_fmaf(qc4[k].w, kc4.w, dot[k]);
-      }
-      kc4 = kn4;
-#pragma unroll
-      for (int k = 0; k < NT; ++k) qc4[k] = qn4[k];
-    }
-#pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      const bool present = c * ATTN_CHUNK + lane < Tk[k];
-      const float sv = present ? dot[k] * scale : -1e9f;
-      const float mc = fmaxf(wave_max_fast(sv), -1e9f);
-      const float e = present ? exp_f32(sv - mc) : 0.0f;
-      const float z = wave_tree_sum_fast(e);
-      sE[k * ESZ + hh * ATTN_CHUNK + lane] = e;
-      if (lane == 0) put_mz(k, hh, make_float2(mc, z));
-    }
-  }
-  // WL (head_dim 64): the weighted sums of head hh run on the wave that
-  // formed its softmax terms, so a wave-level ordering suffices
-  if constexpr (WL) wave_sync();
-  else __syncthreads();
-  // positions 0..nt_k-1 for token k: the first nt_lo for every token, then
-  // the later ones for the tokens that have them
-  int nt[NT];
-#pragma unroll
-  for (int k = 0; k < NT; ++k) nt[k] = min(ATTN_CHUNK, Tk[k] - c * ATTN_CHUNK);
-  int nt_lo = nt[0], nt_hi = nt[0];
-#pragma unroll
-  for (int k = 1; k < NT; ++k) {
-    nt_lo = min(nt_lo, nt[k]);
-    nt_hi = max(nt_hi, nt[k]);
-  }
-#pragma unroll
-  for (int u = 0; u < OPT; ++u) {
-    const int oi = tid + 256 * u;
-    float acc[NT];
-#pragma unroll
-    for (int k = 0; k < NT; ++k) acc[k] = 0.0f;
-    if (oi < gh) {
-      const int hh = oi / hd, i = oi - hh * hd;
-      const float* eh = &sE[hh * ATTN_CHUNK];
-      // positions in groups of 4, the next group's softmax terms and V
-      // values read while this group's fmas run, then the rest one by one
-      const int n4 = nt_lo & ~3;
-      if (n4 > 0) {
-        auto ld4 = [&](int j0, f32x4 (&e4)[NT], f32x4& v4) {
-#pragma unroll
-          for (int k = 0; k < NT; ++k) e4[k] = *reinterpret_cast<const f32x4*>(eh + k * ESZ + j0);
-          v4 = f32x4{sV[j0 * HDM + i], sV[(j0 + 1) * HDM + i], sV[(j0 + 2) * HDM + i], sV[(j0 + 3) * HDM + i]};
-        };
-        f32x4 ec[NT], vcur;
-        ld4(0, ec, vcur);
-#pragma unroll 2
-        for (int j0 = 0; j0 < n4; j0 += 4) {
-          f32x4 en[NT], vnx;
-          ld4(min(j0 + 4, n4 - 4), en, vnx);
-#pragma unroll
-          for (int k = 0; k < NT; ++k) {
-            acc[k] = __builtin_fmaf(ec[k].x, vcur.x, acc[k]);
-            acc[k] = __builtin_fmaf(ec[k].y, vcur.y, acc[k]);
-            acc[k] = __builtin_fmaf(ec[k].z, vcur.z, acc[k]);
-            acc[k] = __builtin_fmaf(ec[k].w, vcur.w, acc[k]);
-          }
-          vcur = vnx;
-#pragma unroll
-          for (int k = 0; k < NT; ++k) ec[k] = en[k];
-        }
-      }
-      for (int j = n4; j < nt_lo; ++j) {
-        const float v = sV[j * HDM + i];
-#pragma unroll
-        for (int k = 0; k < NT; ++k) acc[k] = __builtin_fmaf(eh[k * ESZ + j], v, acc[k]);
-      }
-      for (int j = nt_lo; j < nt_hi; ++j) {
-        const float v = sV[j * HDM + i];
-#pragma unroll
-        for (int k = 0; k < NT; ++k)
-          if (j < nt[k]) acc[k] = __builtin_fmaf(eh[k * ESZ + j], v, acc[k]);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NT; ++k) o[k][u] = acc[k];
-  }
-}
-
 template <int HDM, bool WL>
 __global__ void __launch_bounds__(256) k_attention(const float* __restrict__ q, const float* __restrict__ kc,
                                                    const float* __restrict__ vc, const int* __restrict__ state,
@@ -466,41 +339,38 @@ __global__ void __launch_bounds__(256 * AQ_GROUPS) k_attention_q8k(const float* 
 
 // Prefill: chunk blockIdx.y of kv head blockIdx.x for the tile of tt
 // consecutive tokens from blockIdx.z * tt (token z at position pos0 + z,
-// its own q and partials).  The chunk's K and V rows are staged once; the
-// tile's tokens whose context reaches the chunk then run on it ATTN_TOK at a
-// time (attn_tokens_chunk: for each token the arithmetic of k_attention's
-// launch for that token) and write their partials for the chunk.  Rows the
-// tile stages past a token's context take no part in that token's sums.
-constexpr int ATTN_TOK = 4;
-
-// WL (head_dim 64): every LDS value a wave reads in the token loop (its
-// heads' queries, softmax terms and (m_c, z_c)) was written by the same wave,
-// so the loop orders them within the wave and only the staged K/V rows wait
-// for a work-group barrier.
-template <int HDM, bool WL, int GM>
+// its own q and partials).  The chunk's K and V rows are staged once; a wave
+// then takes 16 rows at a time, a row being one query head of one of the
+// tile's tokens whose context reaches the chunk, and writes their partials.
+//
+// The score chains and the weighted V chains run on v_mfma_f32_16x16x4_f32:
+// its result is the chain of four fmas over k in order, each rounded to
+// nearest even with denormals kept (20 million results over normal, widely
+// spread and denormal operands, none different), so a token's scores and o_c
+// have the bits of the decode attention's fma chains.  Positions past a
+// token's context score -1e9 and weigh 0; a 0 leaves the V chain as it is if
+// that V is finite, so a chunk with an infinity or NaN in V takes the plain
+// chains instead.  Layouts: A lane l holds row l%16, k = l/16; B column l%16, k
+// = l/16; D register i row 4*(l/16) + i, column l%16.  K, V and the softmax
+// terms are stored so that the 64 lanes of an operand read hit 64 banks.
+//
+// Bound by the MFMAs (32 cycles each, 128 per 16 rows and chunk at head_dim
+// 64: 29 us of MFMA time per launch for 1023 tokens, 32 heads); the
+// fma chains it replaces, one lane per (head, position) and (head, dim), took
+// 131 us per launch there, 89 now; 16 heads of 128 over 332 tokens 51.7 -> 24.6).
+template <int HDM, bool FULL>
 __global__ void __launch_bounds__(256) k_attention_tile(const float* __restrict__ q, const float* __restrict__ kc,
                                                         const float* __restrict__ vc, int n_heads, int n_kv_heads,
-                                                        int hd, int max_chunks, float* __restrict__ part_o,
+                                                        int head_dim, int max_chunks, float* __restrict__ part_o,
                                                         float2* __restrict__ part_mz, int pos0, int n_tok, int tt,
                                                         size_t tok_q, size_t tok_o, size_t tok_mz) {
-  // GM 4 (head_dim 64, at most 4 query heads per kv head): sQ and sE for 4
-  // heads, K rows unpadded and swizzled, (m_c, z_c) stored straight from
-  // the wave: 40 KB of LDS, four work groups per CU where the padded layout
-  // for 8 heads (50 KB) fits three
-  constexpr bool SWZ = GM == 4;
-  constexpr int NV = HDM / 16;
-  constexpr int OPT = GM * HDM / 256;
-  constexpr int NQ = GM * HDM / 256;
-  constexpr int KS = SWZ ? HDM : HDM + 4;
-  constexpr int NT = ATTN_TOK;
-  constexpr int QSZ = GM * HDM, ESZ = GM * ATTN_CHUNK;
-  static_assert(!SWZ || (WL && HDM == 64), "the compact layout is for head_dim 64");
-  __shared__ __attribute__((aligned(16))) float sK[ATTN_CHUNK * KS];
+  constexpr int NV = HDM / 16, NS = HDM / 4, ND = HDM / 16;
+  __shared__ __attribute__((aligned(16))) float sK[ATTN_CHUNK * HDM];
   __shared__ __attribute__((aligned(16))) float sV[ATTN_CHUNK * HDM];
-  __shared__ __attribute__((aligned(16))) float sQ[NT * QSZ];
-  __shared__ __attribute__((aligned(16))) float sE[NT * ESZ];
-  __shared__ float2 sMZ[SWZ ? 1 : NT * ATTN_MAX_GROUP];
-  const int tid = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) float s_e[4][16 * ATTN_CHUNK];
+  const int hd = FULL ? HDM : head_dim;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kvh = blockIdx.x, c = blockIdx.y;
   const int z0 = static_cast<int>(blockIdx.z) * tt;
   const int zlo = max(z0, c * ATTN_CHUNK - pos0);  // first token with pos0 + z + 1 > c * ATTN_CHUNK
@@ -509,87 +379,117 @@ __global__ void __launch_bounds__(256) k_attention_tile(const float* __restrict_
   const int group = n_heads / n_kv_heads;
   const int kvd = n_kv_heads * hd;
   const int r4 = hd / 4, nf4 = ATTN_CHUNK * r4;
-  const int gh = group * hd;
   const float scale = 1.0f / sqrtf(static_cast<float>(hd));
-  const size_t head_off = static_cast<size_t>(kvh) * hd;
+  const int rows = (zhi - zlo) * group;
+  // row f is head f % group of token zlo + f / group (f < 2^13, group <= 8:
+  // the product's error stays below one)
+  const uint32_t inv = 65536u / static_cast<uint32_t>(group) + 1u;
+  auto row_token = [&](int f) { return static_cast<int>((static_cast<uint32_t>(f) * inv) >> 16); };
 
   AttnRegs<NV> R;
-  attn_load_chunk<NV>(R, kc, vc, c, pos0 + zhi, kvd, head_off, r4, nf4);
-  // the queries of tokens z .. z+NT-1 (tokens past the tile re-read its last)
-  auto load_q = [&](int z, float (&qv)[NT][NQ]) {
+  attn_load_chunk<NV>(R, kc, vc, c, pos0 + zhi, kvd, static_cast<size_t>(kvh) * hd, r4, nf4);
+  float qa[NS];  // A operands: query row c16 of a row tile, dims 4s + g
+  auto load_q = [&](int rt) {
+    const int f = min(rt * 16 + c16, rows - 1), z = row_token(f);
+    const float* p = q + static_cast<size_t>(zlo + z) * tok_q + static_cast<size_t>(kvh * group + f - z * group) * hd + g;
 #pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      const float* qg = q + static_cast<size_t>(min(z + k, zhi - 1)) * tok_q + static_cast<size_t>(kvh) * gh;
-#pragma unroll
-      for (int u = 0; u < NQ; ++u) qv[k][u] = qg[min(tid + 256 * u, gh - 1)];
-    }
+    for (int s = 0; s < NS; ++s) qa[s] = p[FULL ? 4 * s : 4 * min(s, r4 - 1)];
   };
-  float qv[NT][NQ];
-  load_q(zlo, qv);
+  load_q(wave);
+  // K row j's dims 4s .. 4s+3 at quad s ^ (j % 16), V row j's dims 16d ..
+  // 16d+15 at 16-float group d ^ (j % 4)
+  bool bad = false;
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
     const int f = min(tid + 256 * u, nf4 - 1);
     const int j = f / r4, c4 = f - j * r4;
-    *reinterpret_cast<f32x4*>(&sK[j * KS + (SWZ ? (c4 ^ (j & 15)) : c4) * 4]) = R.k[u];
-    *reinterpret_cast<f32x4*>(&sV[j * HDM + c4 * 4]) = R.v[u];
+    *reinterpret_cast<f32x4*>(&sK[j * HDM + ((c4 ^ (j & 15)) << 2)]) = R.k[u];
+    *reinterpret_cast<f32x4*>(&sV[j * HDM + (((c4 >> 2) ^ (j & 3)) << 4) + ((c4 & 3) << 2)]) = R.v[u];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bad = bad || !(fabsf(R.v[u][i]) <= 3.402823466e38f);
   }
-  if constexpr (WL) __syncthreads();  // the staged rows
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int z = zlo; z < zhi; z += NT) {
-    // the previous tokens' readers of sQ, sE and sMZ are done (and, first, the
-    // staged rows are in)
-    if constexpr (WL) wave_sync();
-    else __syncthreads();
+  float* sE = s_e[wave];
+  const bool wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0;  // of every lane: outside the branch
+  if (lane == 0) sE[0] = wave_bad ? 1.0f : 0.0f;
+  __syncthreads();
+  const bool plain = (s_e[0][0] + s_e[1][0]) + (s_e[2][0] + s_e[3][0]) != 0.0f;
+  __syncthreads();
+  const f32x4 zero4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int rt = wave; rt * 16 < rows; rt += 4) {
+    f32x4 S[4] = {zero4, zero4, zero4, zero4};
 #pragma unroll
-    for (int k = 0; k < NT; ++k) {
+    for (int s = 0; s < NS; ++s) {
 #pragma unroll
-      for (int u = 0; u < NQ; ++u) {
-        const int i = tid + 256 * u;
-        if (i < gh) sQ[k * QSZ + (i / hd) * HDM + i % hd] = qv[k][u];
-      }
+      for (int p = 0; p < 4; ++p)
+        if (FULL || s < r4)
+          S[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[s], sK[(16 * p + c16) * HDM + ((s ^ c16) << 2) + g], S[p], 0, 0, 0);
     }
-    if (z + NT < zhi) load_q(z + NT, qv);
-    if constexpr (WL) wave_sync();
-    else __syncthreads();
-    int Tk[NT];
+    if ((rt + 4) * 16 < rows) load_q(rt + 4);
+    // rows 4g+i of the lane: their positions 16p + c16
+    float* po[4];
+    int nt[4];
 #pragma unroll
-    for (int k = 0; k < NT; ++k) Tk[k] = pos0 + min(z + k, zhi - 1) + 1;
-    float o[NT][OPT];
-    auto put_mz = [&](int k, int hh, float2 v) {
-      if constexpr (SWZ) {
-        if (z + k < zhi)
-          part_mz[static_cast<size_t>(z + k) * tok_mz + static_cast<size_t>(kvh * group + hh) * max_chunks + c] = v;
-      } else {
-        sMZ[k * ATTN_MAX_GROUP + hh] = v;
+    for (int i = 0; i < 4; ++i) {
+      const int f = min(rt * 16 + 4 * g + i, rows - 1), z = row_token(f), h = kvh * group + f - z * group;
+      const size_t pc = static_cast<size_t>(h) * max_chunks + c;
+      po[i] = part_o + static_cast<size_t>(zlo + z) * tok_o + pc * hd;
+      nt[i] = min(ATTN_CHUNK, pos0 + zlo + z + 1 - c * ATTN_CHUNK);
+      float sv[4], e[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) sv[p] = 16 * p + c16 < nt[i] ? S[p][i] * scale : -1e9f;
+      const float mc = fmaxf(row16_max(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]))), -1e9f);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        e[p] = 16 * p + c16 < nt[i] ? exp_f32(sv[p] - mc) : 0.0f;
+        // row r's positions 4s .. 4s+3 at quad s ^ r
+        sE[(4 * g + i) * ATTN_CHUNK + (((4 * p + (c16 >> 2)) ^ (4 * g + i)) << 2) + (c16 & 3)] = e[p];
       }
-    };
-    attn_tokens_chunk<HDM, OPT, NT, WL, GM, SWZ>(sK, sV, sQ, sE, put_mz, c, Tk, group, hd, gh, scale, o);
+      // wave_tree_sum's tree over the 64 positions (slots t and t+32, then
+      // t+16, then within 16), whole on the row's first lane
+      float zs = (e[0] + e[2]) + (e[1] + e[3]);
+      zs = zs + dpp_f<0x108>(zs);
+      zs = zs + dpp_f<0x104>(zs);
+      zs = zs + dpp_f<0x102>(zs);
+      zs = zs + dpp_f<0x101>(zs);
+      if (c16 == 0 && rt * 16 + 4 * g + i < rows) part_mz[static_cast<size_t>(zlo + z) * tok_mz + pc] = make_float2(mc, zs);
+    }
+    wave_sync();
+    const int last = pos0 + zlo + row_token(min(rt * 16 + 15, rows - 1)) + 1 - c * ATTN_CHUNK;  // the tile's longest
+    if (!plain) {
+      f32x4 O[ND];
 #pragma unroll
-    for (int k = 0; k < NT; ++k) {
-      if (z + k < zhi) {
-        float* po = part_o + static_cast<size_t>(z + k) * tok_o;
+      for (int d = 0; d < ND; ++d) O[d] = zero4;
+      const int ns = (min(ATTN_CHUNK, last) + 3) >> 2;
+#pragma unroll 4
+      for (int s = 0; s < ns; ++s) {
+        const float a = sE[c16 * ATTN_CHUNK + ((s ^ c16) << 2) + g];
 #pragma unroll
-        for (int u = 0; u < OPT; ++u) {
-          const int oi = tid + 256 * u;
-          if (oi < gh) {
-            const int hh = oi / hd, i = oi - hh * hd;
-            po[(static_cast<size_t>(kvh * group + hh) * max_chunks + c) * hd + i] = o[k][u];
+        for (int d = 0; d < ND; ++d)
+          O[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sV[(4 * s + g) * HDM + ((d ^ g) << 4) + c16], O[d], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (rt * 16 + 4 * g + i < rows) {
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            if (FULL || 16 * d + c16 < hd) po[i][16 * d + c16] = O[d][i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (rt * 16 + 4 * g + i < rows) {
+          for (int d = c16; d < hd; d += 16) {
+            float acc = 0.0f;
+            for (int j = 0; j < nt[i]; ++j)
+              acc = __builtin_fmaf(sE[(4 * g + i) * ATTN_CHUNK + (((j >> 2) ^ (4 * g + i)) << 2) + (j & 3)],
+                                   sV[j * HDM + (((d >> 4) ^ (j & 3)) << 4) + (d & 15)], acc);
+            po[i][d] = acc;
           }
         }
-        if constexpr (SWZ) {
-          // stored by put_mz
-        } else if constexpr (WL) {
-          // lane 0 of the wave that wrote them: heads wave, wave + 4
-          for (int hh = wave; hh < group; hh += 4)
-            if (lane == 0)
-              part_mz[static_cast<size_t>(z + k) * tok_mz + static_cast<size_t>(kvh * group + hh) * max_chunks + c] =
-                  sMZ[k * ATTN_MAX_GROUP + hh];
-        } else if (tid < group) {
-          part_mz[static_cast<size_t>(z + k) * tok_mz + static_cast<size_t>(kvh * group + tid) * max_chunks + c] =
-              sMZ[k * ATTN_MAX_GROUP + tid];
-        }
       }
     }
+    wave_sync();  // the reads of sE, before the next row tile's terms
   }
 }
 
@@ -675,27 +575,21 @@ hipError_t launch_attention_batch(const float* q, const float* kc, const float* 
     return hipErrorInvalidValue;
   if (n_tok <= 0) return hipSuccess;
   // one work group per (kv head, chunk, token tile); tiles whose tokens do
-  // not reach a chunk return at once
-  // tokens per tile (MCPM_PREFILL_ATTN_TT overrides, a tuning aid)
-  static const int tt_env = [] {
-    const char* v = std::getenv("MCPM_PREFILL_ATTN_TT");
-    return v ? std::atoi(v) : 0;
-  }();
-  const int tt = tt_env >= 1 && tt_env <= 256 ? tt_env : 16;
-  const dim3 grid(n_kv_heads, (pos0 + n_tok - 1) / ATTN_CHUNK + 1, (n_tok + tt - 1) / tt);
+  // not reach a chunk return at once.  A tile is one row tile per wave (64
+  // rows): more per wave, to stage K and V for more tokens, was slower at every
+  // length (1023 tokens, 4 heads per kv head: a prompt in 18.88 ms with 16
+  // tokens, 19.01 with 32, 19.17 with 64; 332 tokens, 8 heads: 7.31 with 8, 8.10
+  // with 32), half of it too beyond 332 tokens (1023: 21.0).
+  const int group = n_heads / n_kv_heads, nch = (pos0 + n_tok - 1) / ATTN_CHUNK + 1;
+  const int tt = (64 + group - 1) / group;
+  const dim3 grid(n_kv_heads, nch, (n_tok + tt - 1) / tt);
   const size_t tok_q = static_cast<size_t>(n_heads) * head_dim;
-  if (head_dim == 64 && n_heads / n_kv_heads <= 4)
-    hipLaunchKernelGGL((k_attention_tile<64, true, 4>), grid, dim3(256), 0, s, q, kc, vc, n_heads, n_kv_heads,
-                       head_dim, max_chunks, part.o, part.mz, pos0, n_tok, tt, tok_q, tok_o, tok_mz);
-  else if (head_dim == 64)
-    hipLaunchKernelGGL((k_attention_tile<64, true, 8>), grid, dim3(256), 0, s, q, kc, vc, n_heads, n_kv_heads, head_dim,
-                       max_chunks, part.o, part.mz, pos0, n_tok, tt, tok_q, tok_o, tok_mz);
-  else if (head_dim < 64)
-    hipLaunchKernelGGL((k_attention_tile<64, false, 8>), grid, dim3(256), 0, s, q, kc, vc, n_heads, n_kv_heads, head_dim,
-                       max_chunks, part.o, part.mz, pos0, n_tok, tt, tok_q, tok_o, tok_mz);
-  else
-    hipLaunchKernelGGL((k_attention_tile<128, false, 8>), grid, dim3(256), 0, s, q, kc, vc, n_heads, n_kv_heads, head_dim,
-                       max_chunks, part.o, part.mz, pos0, n_tok, tt, tok_q, tok_o, tok_mz);
+  auto kern = head_dim == 64    ? k_attention_tile<64, true>
+              : head_dim == 128 ? k_attention_tile<128, true>
+              : head_dim < 64   ? k_attention_tile<64, false>
+                                : k_attention_tile<128, false>;
+  launch_kernel(kern, grid, dim3(256), 0, s, q, kc, vc, n_heads, n_kv_heads, head_dim, max_chunks, part.o, part.mz, pos0,
+                n_tok, tt, tok_q, tok_o, tok_mz);
   return hipGetLastError();
 }
 

@@ -62,6 +62,53 @@ def test_prefill_token_tiles(ctx, case):
     test_prefill_kv_and_tokens_match_per_token(ctx, case)
 
 
+# head_dim 128 and 96 (the attention's instances past 64), 32 (below), groups of 8, 3 and 1 query heads,
+# contexts that end inside a chunk, at its edge and one past it
+ATTN_CASES = [(2, 512, 16, 2, 128, 512, 300, 0, 70), (2, 512, 8, 4, 96, 512, 300, 0, 66), (2, 512, 8, 1, 32, 512, 300, 0, 65),
+              (2, 768, 12, 4, 64, 512, 300, 0, 130), (2, 256, 4, 4, 64, 512, 300, 0, 64), (2, 512, 16, 2, 128, 512, 300, 0, 333)]
+
+
+@pytest.mark.parametrize("case", ATTN_CASES, ids=lambda c: f"h{c[2]}-kv{c[3]}-hd{c[4]}-p{c[8]}")
+def test_prefill_attention_shapes(ctx, case):
+    test_prefill_kv_and_tokens_match_per_token(ctx, case)
+
+
+def test_prefill_infinite_v_leaves_earlier_tokens(ctx):
+    """A V row with infinities weighs 0 in the tokens before it: they keep their bits (0 * inf would be NaN)."""
+    cfg = mcpm.make_config(2, 512, 8, 2, 64, 512, 300)
+    img = mcpm.synth_gguf(cfg, seed=11, mix=0).copy()
+    _, T = O.read_gguf(img)
+    # dimension 0 of the embedding is 0 but for token 299, and layer 0's norm
+    # scales it by 1e38, so that only that token's V overflows; q is 0, so
+    # every score is 0 and the token's K takes no part
+    embd = T["token_embd.weight"][2].reshape(300, 2, 210)
+    embd[:, 0, 0] &= 0xF0
+    embd[:, 0, 128] = (embd[:, 0, 128] & 0xFC) | 2
+    embd[299, 0, 0] |= 0x0F
+    embd[299, 0, 128] |= 3
+    T["blk.0.attn_norm.weight"][2].view(np.float32)[0] = 1e38
+    T["blk.0.attn_q.weight"][2].reshape(-1, 144)[:, :4] = 0
+    T["blk.0.attn_v.weight"][2].reshape(-1, 210)[:, 208:] = np.array([0x2E66], np.uint16).view(np.uint8)  # d = 0.1
+    prompt = np.random.default_rng(5).integers(0, 299, 60).astype(np.int32)
+    prompt[37] = 299
+    eng = mcpm.Engine(ctx, image=img)
+    try:
+        kv = {}
+        for prefill in (False, True):
+            eng.set_prefill(prefill)
+            eng.init_kv_cache(64)
+            eng.generate_greedy(prompt, 1)
+            kv[prefill] = [eng.read_kv(l, 0, 59) for l in range(2)]
+    finally:
+        eng.free()
+    v0 = kv[False][0][1].reshape(59, -1)
+    assert not np.isfinite(v0[37]).all() and np.isfinite(np.delete(v0, 37, axis=0)).all()
+    assert_bits(kv[True][0][1], kv[False][0][1])
+    for i in range(2):
+        assert np.isfinite(kv[False][1][i][:37]).all()
+        assert_bits(kv[True][1][i][:37], kv[False][1][i][:37])
+
+
 def test_prefill_greedy_matches_oracle(ctx):
     cfg = mcpm.make_config(2, 512, 8, 2, 64, 1400, 2000)
     img = mcpm.synth_gguf(cfg, seed=31, mix=0)
