@@ -743,13 +743,18 @@ int prefill_pass(mcpm_engine* e, const int* tokens, int n, int pos0) {
     const GemmRope rp{e->rope, c.head_dim, pos0};
     float* krows = kc + static_cast<size_t>(pos0) * kvd;
     float* vrows = vc + static_cast<size_t>(pos0) * kvd;
+    // (a Q6_K v beside Q4_K q and k: in their launch too)
+    const GemmMore v{view_of(L.wv), kvd, vrows, kvd};
+    const bool with_v = wq.type == MCPM_TYPE_Q4_K && v.w.type == MCPM_TYPE_Q6_K;
     if (wq.type == wk.type && qd % 64 == 0) {
-      MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, &wk, kvd, krows, kvd, &rp));
+      MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, &wk, kvd, krows, kvd, &rp, false,
+                               with_v ? &v : nullptr));
+      if (!with_v) MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, s));
     } else {
       MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, nullptr, 0, nullptr, 0, &rp));
       MCPM_HIP(launch_gemm_q8k(wk, kvd, nbd, n, qb, krows, kvd, false, s, nullptr, 0, nullptr, 0, &rp));
+      MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, s));
     }
-    MCPM_HIP(launch_gemm_q8k(view_of(L.wv), kvd, nbd, n, qb, vrows, kvd, false, s));
     if (l == c.n_layers - 1) break;  // nothing after the last K/V rows reaches the cache
     MCPM_HIP(launch_attention_batch(b.q, kc, vc, c.n_heads, c.n_kv_heads, c.head_dim, e->max_chunks, part, tok_o,
                                     tok_mz, pos0, n, s));

@@ -289,10 +289,11 @@ __device__ __forceinline__ h2 splat2(float v) {
 // of Q6_K, 0.2 of Q4_K) and the first weights from HBM.
 // PF: blocks in flight (loads return in order, so weights and activations are
 // loaded equally far ahead).
+// bid: the work group's index in the GEMM's grid; s_acc: 8*NT*64 entries,
+// one row tile's chains [lane group][token tile][lane].
 template <int WT, int RT, int NT, int PF>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_gemm_q8k(const GemmArgs a) {
+__device__ __forceinline__ void gemm_block(const GemmArgs& a, unsigned bid, f32x4* s_acc) {
   constexpr int NM = (NT + 3) / 4;  // token tiles whose min chain and epilogue a wave takes: w, w+4, ...
-  __shared__ f32x4 s_acc[8 * NT * 64];  // one row tile's chains: [lane group][token tile][lane]
   const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   // Row groups: the first matrix's, then the second's (swiglu: of RT/2 row
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
   // L2), and then an equal share of the r remaining row groups' (row group,
   // token tile) items, so every XCD has the same work; each XCD's L2 keeps
   // about one eighth of the matrix for the whole launch.
-  const int xcd = static_cast<int>(blockIdx.x) & 7, loc = static_cast<int>(blockIdx.x) >> 3;
+  const int xcd = static_cast<int>(bid) & 7, loc = static_cast<int>(bid) >> 3;
   const int n_tt = (a.n_tok + 15) >> 4;
   const int n_tg = (n_tt + NT - 1) / NT;
   const int rq = n_rg >> 3, rr = n_rg & 7;
@@ -605,6 +606,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
   }
 }
 
+template <int WT, int RT, int NT, int PF>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_gemm_q8k(const GemmArgs a) {
+  __shared__ f32x4 s_acc[8 * NT * 64];
+  gemm_block<WT, RT, NT, PF>(a, blockIdx.x, s_acc);
+}
+
+// Two GEMMs on the same activations in one launch, the first grid_a work
+// groups (a multiple of 8, so both keep their XCDs) a Q4_K one (q and k), the
+// rest a Q6_K one (v): v's few rows alone left most CUs idle for 9 us of each
+// layer (32 work groups for 44 tokens).
+template <int RT, int NT, int PF>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
+k_gemm_q4_q6(const GemmArgs a, const GemmArgs b, unsigned grid_a) {
+  __shared__ f32x4 s_acc[8 * NT * 64];
+  if (blockIdx.x < grid_a)
+    gemm_block<0, RT, NT, PF>(a, blockIdx.x, s_acc);
+  else
+    gemm_block<1, RT, NT, PF>(b, blockIdx.x - grid_a, s_acc);
+}
+
 // ------------------------------------------------- attention combine + Q8_K --
 // Per token t (one work group, position pos0 + t): the attention output from
 // the per-token chunk partials -- k_attn_combine's arithmetic for each value:
@@ -706,7 +727,7 @@ hipError_t launch_quant_batch_swiglu(const float* g, const float* u, int ld, int
 
 hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const QuantBatch& q, float* out, int ld_out,
                            bool add, hipStream_t s, const WView* w2, int rows2, float* out2, int ld_out2,
-                           const GemmRope* rope, bool swiglu) {
+                           const GemmRope* rope, bool swiglu, const GemmMore* v) {
   if (w.type != MCPM_TYPE_Q4_K && w.type != MCPM_TYPE_Q6_K) return hipErrorInvalidValue;
   if (rows < 1 || nb < 1 || n_tok < 1) return hipErrorInvalidValue;
   if (rows2 > 0 && (!w2 || w2->type != w.type || (!swiglu && !out2))) return hipErrorInvalidValue;
@@ -719,6 +740,11 @@ hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const Qu
   GemmArgs a{w, rows, nb, n_tok, q.xh, q.xd, q.xbs, out, ld_out, add ? 1 : 0, rows2 > 0 ? *w2 : WView{},
              std::max(rows2, 0), out2, ld_out2, rope ? rope->table : nullptr, rope ? rope->head_dim : 0,
              rope ? rope->pos0 : 0, swiglu ? 1 : 0};
+  // v: a further matrix of the other type, in the same launch
+  const bool pair = v && v->rows > 0;
+  if (pair && (w.type != MCPM_TYPE_Q4_K || v->w.type != MCPM_TYPE_Q6_K || swiglu || add)) return hipErrorInvalidValue;
+  const GemmArgs av{pair ? v->w : WView{}, pair ? v->rows : 0, nb, n_tok, q.xh, q.xd, q.xbs, pair ? v->out : nullptr,
+                    pair ? v->ld_out : 0, 0, WView{}, 0, nullptr, 0, nullptr, 0, 0, 0};
   const bool q4 = w.type == MCPM_TYPE_Q4_K;
   // Token tiles per work group: building a block's weight operands costs about
   // two tiles' chains, so NT token tiles per group cost ceil(tiles / NT) * (2 +
@@ -732,9 +758,10 @@ hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const Qu
     if ((tiles + n - 1) / n * (2 + n) < (tiles + NT - 1) / NT * (2 + NT)) NT = n;
   const int n_tg = (tiles + NT - 1) / NT;
   auto groups = [&](int rpg) { return (rows + rpg - 1) / rpg + (swiglu ? 0 : (std::max(rows2, 0) + rpg - 1) / rpg); };
-  const int RT = swiglu || groups(32) * n_tg >= 256 ? 2 : 1;
-  const int n_rg = groups(swiglu ? 16 : 16 * RT);
-  const dim3 grid(8 * ((n_rg / 8) * n_tg + ((n_rg % 8) * n_tg + 7) / 8));
+  const int RT = swiglu || (groups(32) + (av.rows + 31) / 32) * n_tg >= 256 ? 2 : 1;
+  auto blocks = [&](int n_rg) { return 8u * static_cast<unsigned>((n_rg / 8) * n_tg + ((n_rg % 8) * n_tg + 7) / 8); };
+  const unsigned grid_a = blocks(groups(swiglu ? 16 : 16 * RT));
+  const dim3 grid(grid_a + (pair ? blocks((av.rows + 16 * RT - 1) / (16 * RT)) : 0u));
   // Blocks in flight: two where a block's work is short (few tokens, weights
   // from HBM: 2304 x 5888 Q6_K, 12 tokens, 18.9 us with one, 12.8 with two,
   // 12.6 with four), one where the other wave of the SIMD fills the wait and
@@ -742,7 +769,8 @@ hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const Qu
   // blocks of weights, 20.5 with one).
 #define MCPM_GEMM(R, N, P) \
   if (RT == R && NT == N) { \
-    if (q4) launch_kernel(k_gemm_q8k<0, R, N, P>, grid, dim3(256), 0, s, a); \
+    if (pair) launch_kernel(k_gemm_q4_q6<R, N, P>, grid, dim3(256), 0, s, a, av, grid_a); \
+    else if (q4) launch_kernel(k_gemm_q8k<0, R, N, P>, grid, dim3(256), 0, s, a); \
     else launch_kernel(k_gemm_q8k<1, R, N, P>, grid, dim3(256), 0, s, a); \
   }
   MCPM_GEMM(1, 1, 2) MCPM_GEMM(1, 2, 2) MCPM_GEMM(1, 3, 2) MCPM_GEMM(1, 4, 2)
