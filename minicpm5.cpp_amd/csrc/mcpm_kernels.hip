@@ -642,36 +642,71 @@ hipError_t launch_embedding(const WView& w, const int* state, int dim, float* ou
 
 // ------------------------------------------------- fp32-activation GEMVs ----
 // gemv_f32 (src/ops/ops.cpp:32-43): lane t sums w*x over c = t, t+64, ...
-// (multiply then add), then the 64-lane pairwise tree.  One wave per row; the
-// lane's loads are issued F32_BATCH at a time (the sum then runs over them in
-// order), so a wave keeps 2 * F32_BATCH * 256 bytes in flight where a load
-// per step waited for memory every few terms.  3001 x 2304: 11.8 -> 5.5 us (5.0 TB/s);
-// 8192 x 6144: 34.9 -> 31.8 us (6.3 TB/s); 1000 x 1024: 3.9 us, launch-bound, unchanged.
-constexpr int F32_BATCH = 16;
+// (multiply then add), then the 64-lane pairwise tree.  One wave per row; up to
+// 16 steps' loads are issued together (the sum then runs over them in order),
+// so a wave keeps 2 * 16 * 256 bytes in flight where a load per step waited for
+// memory every few terms.  What a row leaves past whole 16s runs as an 8, a 4
+// and up to four more steps.  The split depends on the column count alone, not
+// on a lane's own column: that sent lanes 0-39 of a row of 1000 through 16 steps
+// together and the others through 15 one by one.  A load per step throughout,
+// split by the lane's column, this: 32768 x 1000 25.5, 47.3, 21.6 us; 8192 x
+// 2047 12.7, 14.2, 12.5; 2304 x 2304 5.4, 3.7, 3.7; 8192 x 5760 32.7, 29.9, 28.9
+// (6.5 TB/s).
+// N steps from column c on.  LAST: the row may end among them (the columns past
+// it read the row's last, unused).
+template <int N, bool LAST = false>
+__device__ __forceinline__ float f32_steps(const float* __restrict__ wr, const float* __restrict__ x, int c, int cols,
+                                           float p) {
+  float wv[N], xv[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) wv[k] = __builtin_nontemporal_load(wr + (LAST ? min(c + 64 * k, cols - 1) : c + 64 * k));
+#pragma unroll
+  for (int k = 0; k < N; ++k) xv[k] = x[LAST ? min(c + 64 * k, cols - 1) : c + 64 * k];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    if (!LAST || c + 64 * k < cols) p = p + wv[k] * xv[k];
+  return p;
+}
 
+// SHORT: rows of at most three steps, one by one (32768 x 64: 3.6 us, 3.9 with
+// the batches in the kernel).
+constexpr int F32_SHORT = 3 * 64;
+
+template <bool SHORT>
 __global__ void __launch_bounds__(256) k_gemv_f32(const float* __restrict__ w, const float* __restrict__ x,
                                                   float* __restrict__ out, int rows, int cols) {
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (r >= rows) return;
   const float* wr = w + static_cast<size_t>(r) * cols;
   float p = 0.0f;
-  int c = lane;
-  for (; c + 64 * (F32_BATCH - 1) < cols; c += 64 * F32_BATCH) {
-    float wv[F32_BATCH], xv[F32_BATCH];
-#pragma unroll
-    for (int k = 0; k < F32_BATCH; ++k) wv[k] = __builtin_nontemporal_load(wr + c + 64 * k);
-#pragma unroll
-    for (int k = 0; k < F32_BATCH; ++k) xv[k] = x[c + 64 * k];
-#pragma unroll
-    for (int k = 0; k < F32_BATCH; ++k) p = p + wv[k] * xv[k];
+  int c = lane, left = cols;
+  if constexpr (!SHORT) {
+    constexpr int S = 64;  // columns a step
+    const int c16 = (cols & ~(16 * S - 1)) + lane;
+    for (; c < c16; c += 16 * S) p = f32_steps<16>(wr, x, c, cols, p);
+    left = cols & (16 * S - 1);
+    if (left >= 8 * S) {
+      p = f32_steps<8>(wr, x, c, cols, p);
+      c += 8 * S;
+      left -= 8 * S;
+    }
+    if (left >= 4 * S) {
+      p = f32_steps<4>(wr, x, c, cols, p);
+      c += 4 * S;
+      left -= 4 * S;
+    }
   }
-  for (; c < cols; c += 64) p = p + wr[c] * x[c];
+  if (!SHORT && left > 2 * 64)
+    p = f32_steps<4, true>(wr, x, c, cols, p);
+  else
+    for (; c < cols; c += 64) p = p + wr[c] * x[c];
   p = wave_tree_sum(p);
   if (lane == 0) out[r] = p;
 }
 
 hipError_t launch_gemv_f32(const float* w, const float* x, float* out, int rows, int cols, hipStream_t s) {
-  hipLaunchKernelGGL(k_gemv_f32, dim3((rows + 3) / 4), dim3(256), 0, s, w, x, out, rows, cols);
+  hipLaunchKernelGGL(cols <= F32_SHORT ? k_gemv_f32<true> : k_gemv_f32<false>, dim3((rows + 3) / 4), dim3(256), 0, s, w,
+                     x, out, rows, cols);
   return hipGetLastError();
 }
 

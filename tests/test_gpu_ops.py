@@ -294,6 +294,14 @@ def test_gemv_f32_activations_bit_exact(ctx, orc, gtype, rows, cols, off):
     assert_bits(ctx.download(od, np.float32, rows), want)
 
 
+# F32 rows around the kernel's steps: at most three 64-column steps, one column past them, the remainders of
+# 8, 4, 2 and 1 steps with and without a ragged last one, and more rows than work groups run at once
+@pytest.mark.parametrize("rows,cols", [(5, 64), (5, 192), (7, 193), (6, 255), (5, 256), (6, 321), (7, 449), (9, 511), (5, 512),
+                                       (3, 705), (6, 897), (2050, 1000), (5, 1024 + 640), (6, 2048 + 257)])
+def test_gemv_f32_steps(ctx, orc, rows, cols):
+    test_gemv_f32_activations_bit_exact(ctx, orc, mcpm.TYPE_F32, rows, cols, 1)
+
+
 def test_unsupported_type_rejected(ctx):
     with pytest.raises(mcpm.McpmError) as ei:
         ctx.tensor(np.zeros(256 * 2, np.uint8), 1, 256, 1)  # F16
