@@ -487,7 +487,7 @@ int mcpm_gemv_q8_0(mcpm_ctx* c, const mcpm_tensor* w, const float* x, float* out
   if (!c || !w || !x || !out) return fail(MCPM_ERR_ARG, "mcpm_gemv_q8_0: null argument");
   if (w->t.type != MCPM_TYPE_Q8_0) return fail(MCPM_ERR_UNSUPPORTED, "mcpm_gemv_q8_0: wrong tensor type");
   if (cols != w->t.cols || rows <= 0 || rows > w->t.rows) return fail(MCPM_ERR_ARG, "mcpm_gemv_q8_0: bad shape");
-  MCPM_HIP(launch_gemv_q8_0(view_of(w->t), x, out, rows, cols, c->stream));
+  MCPM_HIP(launch_gemv_q8_0(view_of(w->t), x, out, rows, cols, c->n_cu, c->stream));
   return MCPM_OK;
 }
 

@@ -741,27 +741,27 @@ hipError_t launch_stream_read(const void* src, size_t bytes, int grid, uint32_t*
 // (i ascending, multiply then add); row = row + s*d over blocks in order.
 //
 // The blocks' sums s do not depend on each other, only the row chain does: a
-// lane takes one (row, block), a work group Q80_ROWS rows and 256 / Q80_ROWS
-// blocks a step, and leaves s*d in LDS; after up to Q80_CHUNK blocks one lane
-// per row runs the chain over them.  Consecutive lanes take consecutive rows,
-// whose 32-byte codes are consecutive (256-byte runs).  8 rows a work group:
-// 288 work groups at 2304 rows.  Bound by load latency (14 MB take 2.7 us at the copy
-// rate).  One lane per whole row gave 9 work groups at 2304 rows: 2304 x 5760 52.7 -> 7.6 us,
-// 1000 x 1024 10.8 -> 3.8, 8192 x 6144 87.0 -> 20.9 (53.7 MB, 2.6 TB/s).
-constexpr int Q80_ROWS = 8, Q80_PAR = 256 / Q80_ROWS, Q80_CHUNK = 256;
-
+// lane takes one (row, block), a work group ROWS rows and 256 / ROWS blocks a
+// step, and leaves s*d in LDS; after up to 2048 / ROWS blocks one lane per row
+// runs the chain over them.  Consecutive lanes take consecutive rows, whose
+// 32-byte codes are consecutive (256-byte runs with 8 rows).  8 rows a work
+// group: 288 work groups at 2304 rows.  Bound by load latency.  One lane per
+// whole row gave 9 work groups at 2304 rows: 2304 x 5760 52.7 -> 7.6 us, 1000 x
+// 1024 10.8 -> 3.8, 8192 x 6144 87.0 -> 20.9 (53.7 MB, 2.6 TB/s).
+template <int ROWS>
 __global__ void __launch_bounds__(256) k_gemv_q8_0(const WView w, const float* __restrict__ x,
                                                    float* __restrict__ out, int rows, int cols) {
-  __shared__ float sp[Q80_ROWS][Q80_CHUNK + 1];
-  const int tid = threadIdx.x, rr = tid % Q80_ROWS, bl = tid / Q80_ROWS;
-  const int r = blockIdx.x * Q80_ROWS + rr;
+  constexpr int PAR = 256 / ROWS, CHUNK = 2048 / ROWS;
+  __shared__ float sp[ROWS][CHUNK + 1];
+  const int tid = threadIdx.x, rr = tid % ROWS, bl = tid / ROWS;
+  const int r = blockIdx.x * ROWS + rr;
   const int rc = min(r, rows - 1);  // lanes past the last row repeat it (unused)
   const int nb = cols / QK8_0;
   float row = 0.0f;
-  for (int c0 = 0; c0 < nb; c0 += Q80_CHUNK) {
-    const int c1 = min(c0 + Q80_CHUNK, nb);
+  for (int c0 = 0; c0 < nb; c0 += CHUNK) {
+    const int c1 = min(c0 + CHUNK, nb);
 #pragma unroll 2
-    for (int b = c0 + bl; b < c1; b += Q80_PAR) {
+    for (int b = c0 + bl; b < c1; b += PAR) {
       const size_t blk = static_cast<size_t>(b) * w.rows + rc;
       u32x4 q4[2];
       q4[0] = ld_stream4(w.p0 + blk * 32);
@@ -780,17 +780,47 @@ __global__ void __launch_bounds__(256) k_gemv_q8_0(const WView w, const float* _
       sp[rr][b - c0] = s * fp16_to_fp32(dh);
     }
     __syncthreads();
-    if (tid < Q80_ROWS) {
+    if (tid < ROWS) {
 #pragma unroll 8
       for (int b = 0; b < c1 - c0; ++b) row = row + sp[tid][b];
     }
     __syncthreads();  // the chain's reads before the next blocks' products
   }
-  if (tid < Q80_ROWS && r < rows) out[r] = row;
+  if (tid < ROWS && r < rows) out[r] = row;
 }
 
-hipError_t launch_gemv_q8_0(const WView& w, const float* x, float* out, int rows, int cols, hipStream_t s) {
-  hipLaunchKernelGGL(k_gemv_q8_0, dim3((rows + Q80_ROWS - 1) / Q80_ROWS), dim3(256), 0, s, w, x, out, rows, cols);
+// One lane per row: no LDS, no barrier, and x by scalar loads.
+__global__ void __launch_bounds__(256) k_gemv_q8_0_rows(const WView w, const float* __restrict__ x,
+                                                        float* __restrict__ out, int rows, int cols) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= rows) return;
+  const int nb = cols / QK8_0;
+  float row = 0.0f;
+  for (int b = 0; b < nb; ++b) {
+    const size_t blk = static_cast<size_t>(b) * w.rows + r;
+    const int8_t* q = reinterpret_cast<const int8_t*>(w.p0 + blk * 32);
+    float s = 0.0f;
+    for (int i = 0; i < QK8_0; ++i) s = s + static_cast<float>(q[i]) * x[b * QK8_0 + i];
+    const uint16_t dh = w.p1[blk * 2] | (w.p1[blk * 2 + 1] << 8);
+    row = row + s * fp16_to_fp32(dh);
+  }
+  out[r] = row;
+}
+
+// The more rows, the more of the chip they fill by themselves, and the less the
+// split of a row's blocks is worth its barrier.  A lane per row where that is a
+// wave for every SIMD (64 rows each; 65,536 rows on 256 CUs): 130560 x 1536 31.2
+// us, with 8 rows a work group 64.4, with 32 50.7; 65536 x 2304 35.7, 54.5, 44.7
+// (weights in the Infinity Cache; from HBM 50.0, 55.3, 45.8).  32 rows a work
+// group where that is one for every CU: 32768 x 2304 21.9 us, with 8 rows 27.1,
+// a lane per row 33.9; 12000 x 1024 6.1, 6.5, 10.8; 8192 x 2304 9.7, 9.2, 21.8.
+hipError_t launch_gemv_q8_0(const WView& w, const float* x, float* out, int rows, int cols, int n_cu, hipStream_t s) {
+  if (rows >= 256 * n_cu)
+    hipLaunchKernelGGL(k_gemv_q8_0_rows, dim3((rows + 255) / 256), dim3(256), 0, s, w, x, out, rows, cols);
+  else if (rows > 32 * n_cu)
+    hipLaunchKernelGGL(k_gemv_q8_0<32>, dim3((rows + 31) / 32), dim3(256), 0, s, w, x, out, rows, cols);
+  else
+    hipLaunchKernelGGL(k_gemv_q8_0<8>, dim3((rows + 7) / 8), dim3(256), 0, s, w, x, out, rows, cols);
   return hipGetLastError();
 }
 

@@ -302,6 +302,13 @@ def test_gemv_f32_steps(ctx, orc, rows, cols):
     test_gemv_f32_activations_bit_exact(ctx, orc, mcpm.TYPE_F32, rows, cols, 1)
 
 
+# Q8_0 rows around the kernel's splits on 256 CUs: 8 rows a work group up to 8192 rows, 32 past that (its
+# 64-block chunks whole, one past them, and ragged last work groups), a lane per row from 65536 on
+@pytest.mark.parametrize("rows,cols", [(8192, 32), (8193, 96), (8193, 64 * 32), (8200, 65 * 32), (65535, 32), (65536, 64), (70001, 96)])
+def test_gemv_q8_0_splits(ctx, orc, rows, cols):
+    test_gemv_f32_activations_bit_exact(ctx, orc, mcpm.TYPE_Q8_0, rows, cols, 1)
+
+
 def test_unsupported_type_rejected(ctx):
     with pytest.raises(mcpm.McpmError) as ei:
         ctx.tensor(np.zeros(256 * 2, np.uint8), 1, 256, 1)  # F16
