@@ -93,7 +93,11 @@ hipError_t launch_quantize_q8k(const float* x, const float* gamma, float eps, in
 // rmsnorm (src/ops/ops.cpp:468-481): out = (x*rms)*w.  One work group, which
 // reads all of x before it writes (out may be x).  Up to NV values a thread
 // stay in registers with their weights, so the vector is read once; the
-// second trip to memory is for longer ones only (2304 values: 4.1 -> 3.1 us).
+// second trip to memory is for longer ones only (2304 values: 4.1 -> 3.1 us),
+// whose values past those are loaded NV at a time in both passes (a load a step:
+// 16384 values 13.9 us, 262144 226; now 7.4 and 93).  A batch that passes the end
+// reads the thread's own first value of it again, never another thread's (which
+// out may have overwritten).
 template <int NV>
 __global__ void __launch_bounds__(256) k_rmsnorm(const float* x, const float* __restrict__ w, float eps, int dim,
                                                  float* out) {
@@ -109,12 +113,30 @@ __global__ void __launch_bounds__(256) k_rmsnorm(const float* x, const float* __
 #pragma unroll
   for (int k = 0; k < NV; ++k)
     if (tid + 256 * k < dim) p = p + v[k] * v[k];
-  for (int i = tid + 256 * NV; i < dim; i += 256) p = p + x[i] * x[i];
+  for (int i = tid + 256 * NV; i < dim; i += 256 * NV) {
+    float y[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) y[k] = x[i + 256 * k < dim ? i + 256 * k : i];
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (i + 256 * k < dim) p = p + y[k] * y[k];
+  }
   const float rms = block_rms_1sync(p, dim, eps, red);
 #pragma unroll
   for (int k = 0; k < NV; ++k)
     if (tid + 256 * k < dim) out[tid + 256 * k] = (v[k] * rms) * g[k];
-  for (int i = tid + 256 * NV; i < dim; i += 256) out[i] = (x[i] * rms) * w[i];
+  for (int i = tid + 256 * NV; i < dim; i += 256 * NV) {
+    float y[NV], h[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const int j = i + 256 * k < dim ? i + 256 * k : i;
+      y[k] = x[j];
+      h[k] = w[j];
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (i + 256 * k < dim) out[i + 256 * k] = (y[k] * rms) * h[k];
+  }
 }
 
 hipError_t launch_rmsnorm(const float* x, const float* w, float eps, int dim, float* out, hipStream_t s) {

@@ -133,8 +133,9 @@ def test_rmsnorm_ops(ctx, orc, dim):
     assert_bits(ctx.download(qd, mcpm.Q8_K, dim // 256), wq)
 
 
-# fewer values than threads, one past the 3072 a work group keeps in registers, a ragged tail; out is x
-@pytest.mark.parametrize("dim", [1, 255, 3073, 6000])
+# fewer values than threads, one past the 3072 a work group keeps in registers, a ragged tail, whole
+# batches of 3072 past them, one value and a ragged batch past those; out is x
+@pytest.mark.parametrize("dim", [1, 255, 3073, 6000, 6144, 6145, 20011])
 def test_rmsnorm_in_place(ctx, orc, dim):
     rng = np.random.default_rng(dim)
     x, w = rand_act(rng, dim, 2.0), rand_act(rng, dim, 1.0)
