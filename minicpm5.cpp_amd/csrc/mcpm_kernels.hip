@@ -521,8 +521,10 @@ __global__ void __launch_bounds__(256) k_attention_tile(const float* __restrict_
 // Lane c holds chunk c's (m_c, z_c) and forms f_c once for the wave (each
 // output formed every f_c itself before, an exp between each two loads); the
 // chains read it by lane, and the o_c of COMBINE_BATCH chunks are loaded
-// together.  Average over 32 heads of 64 at 9 chunks and 16 of 128 at 63: 22.9 ->
-// 4.5 us.
+// together, the first ones before the maximum (one chunk has nothing else to
+// wait for: 64 heads of 64 at up to 64 positions, a decoded layer 51.1 -> 50.8 us,
+// 50.2 with a thread per output and no lane moves).  Average over 32 heads of 64
+// at 9 chunks and 16 of 128 at 63: 22.9 -> 4.5 us.
 constexpr int COMBINE_BATCH = 16;
 
 __global__ void __launch_bounds__(64) k_attn_combine(const float* __restrict__ part_o,
@@ -537,6 +539,12 @@ __global__ void __launch_bounds__(64) k_attn_combine(const float* __restrict__ p
   // lanes past the last chunk hold it again: the maximum is unchanged, and
   // the chains stop before them
   float2 cur = mz[min(lane, nch - 1)];
+  float ov[COMBINE_BATCH];
+  auto load_o = [&](int c) {
+#pragma unroll
+    for (int k = 0; k < COMBINE_BATCH; ++k) ov[k] = o[static_cast<size_t>(min(c + k, nch - 1)) * hd];
+  };
+  load_o(0);  // in flight beside the maximum
   float m = cur.x;
   for (int c0 = 64; c0 < nch; c0 += 64) m = fmaxf(m, mz[min(c0 + lane, nch - 1)].x);
   m = wave_max_fast(m);
@@ -546,9 +554,7 @@ __global__ void __launch_bounds__(64) k_attn_combine(const float* __restrict__ p
     const float f = exp_f32(cur.x - m);
     const int n = min(64, nch - c0);
     for (int j0 = 0; j0 < n; j0 += COMBINE_BATCH) {
-      float ov[COMBINE_BATCH];
-#pragma unroll
-      for (int k = 0; k < COMBINE_BATCH; ++k) ov[k] = o[static_cast<size_t>(min(c0 + j0 + k, nch - 1)) * hd];
+      if (c0 + j0 > 0) load_o(c0 + j0);
 #pragma unroll
       for (int k = 0; k < COMBINE_BATCH; ++k) {
         if (j0 + k < n) {  // uniform
