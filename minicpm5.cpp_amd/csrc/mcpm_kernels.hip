@@ -603,13 +603,16 @@ hipError_t launch_attention_batch(const float* q, const float* kc, const float* 
     return hipErrorInvalidValue;
   if (n_tok <= 0) return hipSuccess;
   // one work group per (kv head, chunk, token tile); tiles whose tokens do
-  // not reach a chunk return at once.  A tile is one row tile per wave (64
-  // rows): more per wave, to stage K and V for more tokens, was slower at every
-  // length (1023 tokens, 4 heads per kv head: a prompt in 18.88 ms with 16
-  // tokens, 19.01 with 32, 19.17 with 64; 332 tokens, 8 heads: 7.31 with 8, 8.10
-  // with 32), half of it too beyond 332 tokens (1023: 21.0).
+  // not reach a chunk return at once.  A tile is the whole tokens of one row tile
+  // per wave, 64 rows at most: more rows per wave, to stage K and V for more
+  // tokens, were slower at every length (1023 tokens, 4 heads per kv head: a
+  // prompt in 18.88 ms with 16 tokens, 19.01 with 32, 19.17 with 64; 332 tokens, 8
+  // heads: 7.31 with 8, 8.10 with 32), half of it too beyond 332 tokens (1023:
+  // 21.0).  Rounded up instead, groups of 3, 5, 6 and 7 heads gave one wave a
+  // second row tile of 1 to 6 rows (four layers, 7 heads of 128 per kv head, 1023
+  // tokens: 1681 us, 1440 rounded down; 3 heads of 64: 531, 482).
   const int group = n_heads / n_kv_heads, nch = (pos0 + n_tok - 1) / ATTN_CHUNK + 1;
-  const int tt = (64 + group - 1) / group;
+  const int tt = 64 / group;
   const dim3 grid(n_kv_heads, nch, (n_tok + tt - 1) / tt);
   const size_t tok_q = static_cast<size_t>(n_heads) * head_dim;
   auto kern = head_dim == 64    ? k_attention_tile<64, true>

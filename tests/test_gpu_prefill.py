@@ -66,6 +66,8 @@ def test_prefill_token_tiles(ctx, case):
 # contexts that end inside a chunk, at its edge and one past it
 ATTN_CASES = [(2, 512, 16, 2, 128, 512, 300, 0, 70), (2, 512, 8, 4, 96, 512, 300, 0, 66), (2, 512, 8, 1, 32, 512, 300, 0, 65),
               (2, 768, 12, 4, 64, 512, 300, 0, 130), (2, 256, 4, 4, 64, 512, 300, 0, 64), (2, 512, 16, 2, 128, 512, 300, 0, 333)]
+# groups that do not divide a wave's 16 rows: 5, 6 and 7 query heads, a last token tile that is not full
+ATTN_CASES += [(2, 512, 20, 4, 64, 512, 300, 0, 90), (2, 512, 24, 4, 64, 512, 300, 0, 131), (2, 512, 28, 4, 64, 512, 300, 0, 77)]
 
 
 @pytest.mark.parametrize("case", ATTN_CASES, ids=lambda c: f"h{c[2]}-kv{c[3]}-hd{c[4]}-p{c[8]}")
