@@ -43,7 +43,7 @@ struct TimedPair {
 struct PrefillBufs {
   int cap = 0, max_chunks = 0;
   int* tokens = nullptr;
-  float *x = nullptr, *q = nullptr, *g = nullptr, *u = nullptr, *part = nullptr;
+  float *x = nullptr, *q = nullptr, *g = nullptr, *part = nullptr;
   _Float16 *xh = nullptr, *xbs = nullptr;
   float* xd = nullptr;
 };
@@ -173,7 +173,7 @@ void drop_graph(mcpm_engine* e) {
 void free_prefill(PrefillBufs& b) {
   for (void* p : {static_cast<void*>(b.tokens), static_cast<void*>(b.x),
                   static_cast<void*>(b.q), static_cast<void*>(b.g),
-                  static_cast<void*>(b.u), static_cast<void*>(b.part), static_cast<void*>(b.xh),
+                  static_cast<void*>(b.part), static_cast<void*>(b.xh),
                   static_cast<void*>(b.xbs), static_cast<void*>(b.xd)})
     if (p) (void)hipFree(p);
   b = PrefillBufs{};
@@ -699,10 +699,10 @@ int ensure_prefill(mcpm_engine* e, int cap) {
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.x), n * c.dim * 4);
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.q), n * qd * 4);
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.g), n * c.ffn * 4);
-  if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.u), n * c.ffn * 4);
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.part), n * c.n_heads * e->max_chunks * (c.head_dim + 2) * 4);
   // quantized activations: whole tiles of 16 tokens, and the 16 bytes a GEMM
-  // lane may read past the last bsums
+  // lane may read past the last bsums (zeroed by alloc_dev, as they must be:
+  // QuantBatch)
   const size_t nt = (n + 15) / 16 * 16;
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xh), nt * kmax * 2);
   if (!rc) rc = alloc_dev(reinterpret_cast<void**>(&b.xd), nt * (kmax / QK_K) * 4);
@@ -735,41 +735,28 @@ int prefill_pass(mcpm_engine* e, const int* tokens, int n, int pos0) {
     float* kc = e->kc + static_cast<size_t>(l) * e->max_seq * kvd;
     float* vc = e->vc + static_cast<size_t>(l) * e->max_seq * kvd;
     const int nbd = c.dim / QK_K;
-    MCPM_HIP(launch_quant_batch(b.x, nullptr, c.dim, L.attn_norm, c.eps, c.dim, c.dim, PRO_NORM_AWAY, n, qb, s));
+    MCPM_HIP(launch_quant_batch(b.x, c.dim, L.attn_norm, c.eps, c.dim, c.dim, PRO_NORM_AWAY, n, qb, s));
     // q rotated into b.q and k rotated into the cache rows by the GEMM's
-    // RoPE epilogue, in one launch when q and k share a type (q's rows a
-    // multiple of 64); v straight into the cache rows
+    // RoPE epilogue, in one launch (both are Q4_K), with a Q6_K v straight into
+    // its cache rows; a Q4_K v has a launch of its own
     const WView wq = view_of(L.wq), wk = view_of(L.wk), wg = view_of(L.wg), wu = view_of(L.wu);
     const GemmRope rp{e->rope, c.head_dim, pos0};
     float* krows = kc + static_cast<size_t>(pos0) * kvd;
     float* vrows = vc + static_cast<size_t>(pos0) * kvd;
-    // (a Q6_K v beside Q4_K q and k: in their launch too)
     const GemmMore v{view_of(L.wv), kvd, vrows, kvd};
-    const bool with_v = wq.type == MCPM_TYPE_Q4_K && v.w.type == MCPM_TYPE_Q6_K;
-    if (wq.type == wk.type && qd % 64 == 0) {
-      MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, &wk, kvd, krows, kvd, &rp, false,
-                               with_v ? &v : nullptr));
-      if (!with_v) MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, s));
-    } else {
-      MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, nullptr, 0, nullptr, 0, &rp));
-      MCPM_HIP(launch_gemm_q8k(wk, kvd, nbd, n, qb, krows, kvd, false, s, nullptr, 0, nullptr, 0, &rp));
-      MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, s));
-    }
+    const bool with_v = v.w.type == MCPM_TYPE_Q6_K;
+    MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, &wk, kvd, krows, kvd, &rp, false,
+                             with_v ? &v : nullptr));
+    if (!with_v) MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, s));
     if (l == c.n_layers - 1) break;  // nothing after the last K/V rows reaches the cache
     MCPM_HIP(launch_attention_batch(b.q, kc, vc, c.n_heads, c.n_kv_heads, c.head_dim, e->max_chunks, part, tok_o,
                                     tok_mz, pos0, n, s));
     MCPM_HIP(launch_quant_batch_attn(part, tok_o, tok_mz, pos0, n, c.n_heads, c.head_dim, e->max_chunks, qb, s));
     MCPM_HIP(launch_gemm_q8k(view_of(L.wo), c.dim, qd / QK_K, n, qb, b.x, c.dim, true, s));
-    MCPM_HIP(launch_quant_batch(b.x, nullptr, c.dim, L.ffn_norm, c.eps, c.dim, c.dim, PRO_NORM_AWAY, n, qb, s));
-    if (wg.type == wu.type && c.ffn % 64 == 0) {
-      // gate and up in one launch, h = silu(gate)*up written by its epilogue
-      MCPM_HIP(launch_gemm_q8k(wg, c.ffn, nbd, n, qb, b.g, c.ffn, false, s, &wu, c.ffn, nullptr, 0, nullptr, true));
-      MCPM_HIP(launch_quant_batch(b.g, nullptr, c.ffn, nullptr, 0.0f, c.ffn_pad, c.ffn, PRO_QUANT_AWAY, n, qb, s));
-    } else {
-      MCPM_HIP(launch_gemm_q8k(wg, c.ffn, nbd, n, qb, b.g, c.ffn, false, s));
-      MCPM_HIP(launch_gemm_q8k(wu, c.ffn, nbd, n, qb, b.u, c.ffn, false, s));
-      MCPM_HIP(launch_quant_batch_swiglu(b.g, b.u, c.ffn, c.ffn, c.ffn_pad, n, qb, s));
-    }
+    MCPM_HIP(launch_quant_batch(b.x, c.dim, L.ffn_norm, c.eps, c.dim, c.dim, PRO_NORM_AWAY, n, qb, s));
+    // gate and up in one launch, h = silu(gate)*up written by its epilogue
+    MCPM_HIP(launch_gemm_q8k(wg, c.ffn, nbd, n, qb, b.g, c.ffn, false, s, &wu, c.ffn, nullptr, 0, nullptr, true));
+    MCPM_HIP(launch_quant_batch(b.g, c.ffn, nullptr, 0.0f, c.ffn_pad, c.ffn, PRO_QUANT_AWAY, n, qb, s));
     MCPM_HIP(launch_gemm_q8k(view_of(L.wd), c.dim, c.ffn_pad / QK_K, n, qb, b.x, c.dim, true, s));
   }
   return MCPM_OK;

@@ -346,17 +346,17 @@ hipError_t launch_attn_combine(const AttnPart& part, const int* state, int n_hea
 // ---- prefill (batched prompt tokens; csrc/mcpm_prefill.hip) ----
 // Per-token Q8_K activations in tiles of 16 tokens (the last one whole): fp16
 // codes in the GEMM's operand order, d [tile][dim/256][16], fp16 bsums
-// [tile][dim/256][16][16] and 16 readable bytes after them.
+// [tile][dim/256][16][16] and 16 readable bytes after them.  Allocated zeroed:
+// the GEMM multiplies what lies past a token's last bsums (a token slot not
+// written yet, or those 16 bytes) by 0, so it has to be finite.
 struct QuantBatch {
   _Float16* xh;
   float* xd;
   _Float16* xbs;
 };
 hipError_t launch_embed_batch(const WView& w, const int* tokens, int n_tok, int dim, float* x, hipStream_t s);
-hipError_t launch_quant_batch(const float* x, const float* u, int ld_x, const float* gamma, float eps, int dim,
-                              int n_valid, int mode, int n_tok, QuantBatch q, hipStream_t s);
-hipError_t launch_quant_batch_swiglu(const float* g, const float* u, int ld, int n_valid, int dim, int n_tok,
-                                     QuantBatch q, hipStream_t s);
+hipError_t launch_quant_batch(const float* x, int ld_x, const float* gamma, float eps, int dim, int n_valid, int mode,
+                              int n_tok, QuantBatch q, hipStream_t s);
 // RoPE applied to a GEMM's row pairs before they are stored: the (cos, sin)
 // table (head_dim/2 pairs per position), token t at position pos0 + t.
 struct GemmRope {

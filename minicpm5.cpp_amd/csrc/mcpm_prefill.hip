@@ -51,12 +51,9 @@ __global__ void __launch_bounds__(256) k_embed_batch(const WView w, const int* _
 
 // ------------------------------------------------------------- quantize ----
 // Per token (one work group each): the Q8_K quantization of the GEMV
-// prologues, written as fp16 codes [t][K], d [t][nb] and fp16 bsums
-// [t][nb][16].  mode: PRO_QUANT_EVEN / PRO_QUANT_AWAY / PRO_NORM_AWAY /
-// PRO_NORM_EVEN, or QB_SWIGLU: v = silu(g)*u (decode's gate/up epilogue) for
-// i < n_valid and 0 beyond, then ties-away (decode's down prologue).
-constexpr int QB_SWIGLU = 100;
-
+// prologues, written as the GEMM's operands (store_codes).  mode:
+// PRO_QUANT_EVEN / PRO_QUANT_AWAY / PRO_NORM_AWAY / PRO_NORM_EVEN; values from
+// n_valid on quantize as 0.
 // The quantized activations in the order the GEMM's MFMA operands want them,
 // in tiles of 16 tokens: codes [tile][block][lane group m][K-half g][token of
 // the tile][8 halves], the 8 halves being elements 64g + 4m .. +3 and 64g + 32
@@ -89,8 +86,8 @@ __device__ __forceinline__ int quant_token(unsigned b) {
 }
 static dim3 quant_grid(int n_tok) { return dim3(128 * ((n_tok + 127) / 128)); }
 
-__global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x, const float* __restrict__ u,
-                                                     int ld_x, const float* __restrict__ gamma, float eps, int dim,
+__global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x, int ld_x,
+                                                     const float* __restrict__ gamma, float eps, int dim,
                                                      int n_valid, int mode, int n_tok, _Float16* __restrict__ xh,
                                                      float* __restrict__ xd, _Float16* __restrict__ xbs) {
   __shared__ float red[260];
@@ -98,9 +95,8 @@ __global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x
   if (t >= n_tok) return;  // uniform, before any barrier
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float* xt = x + static_cast<size_t>(t) * ld_x;
-  const float* ut = u ? u + static_cast<size_t>(t) * ld_x : nullptr;
   const bool norm = (mode == PRO_NORM_AWAY || mode == PRO_NORM_EVEN);
-  const bool away = (mode == PRO_QUANT_AWAY || mode == PRO_NORM_AWAY || mode == QB_SWIGLU);
+  const bool away = (mode == PRO_QUANT_AWAY || mode == PRO_NORM_AWAY);
   float rms = 1.0f;
   if (norm) rms = block_rms_scale(xt, dim, eps, red);
   const int nb = dim / QK_K;
@@ -109,18 +105,8 @@ __global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const int i = b * QK_K + 4 * lane + k;
-      if (mode == QB_SWIGLU) {
-        float h = 0.0f;
-        if (i < n_valid) {
-          const float g = xt[i];
-          const float silu = g / (1.0f + exp_f32(-g));
-          h = silu * ut[i];
-        }
-        v[k] = h;
-      } else {
-        v[k] = i < n_valid ? xt[i] : 0.0f;
-        if (norm) v[k] = (v[k] * rms) * gamma[i];
-      }
+      v[k] = i < n_valid ? xt[i] : 0.0f;
+      if (norm) v[k] = (v[k] * rms) * gamma[i];
     }
     uint32_t packed;
     float d;
@@ -132,13 +118,13 @@ __global__ void __launch_bounds__(256) k_quant_batch(const float* __restrict__ x
 
 // k_quant_batch for up to 4*MAXB blocks per token, with every global load
 // issued at the start: wave w holds blocks w, w+4, ... (lane l: values 4l ..
-// 4l+3 of each, with their gamma or u), RMSNorm's strided partials are read
+// 4l+3 of each, with their gamma), RMSNorm's strided partials are read
 // back from an LDS copy of the row (thread t: x[t], x[t+256], ... in order,
 // as block_rms_scale sums them), and each block is quantized from registers.
 // Same operations and outputs as k_quant_batch.
 template <int MAXB>
-__global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__ x, const float* __restrict__ u,
-                                                       int ld_x, const float* __restrict__ gamma, float eps, int dim,
+__global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__ x, int ld_x,
+                                                       const float* __restrict__ gamma, float eps, int dim,
                                                        int n_valid, int mode, int n_tok, _Float16* __restrict__ xh,
                                                        float* __restrict__ xd, _Float16* __restrict__ xbs) {
   __shared__ float red[260];
@@ -147,21 +133,18 @@ __global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__
   if (t >= n_tok) return;  // uniform, before any barrier
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const float* xt = x + static_cast<size_t>(t) * ld_x;
-  const float* ut = u ? u + static_cast<size_t>(t) * ld_x : nullptr;
   const bool norm = (mode == PRO_NORM_AWAY || mode == PRO_NORM_EVEN);
-  const bool swiglu = mode == QB_SWIGLU;
-  const bool away = (mode == PRO_QUANT_AWAY || mode == PRO_NORM_AWAY || swiglu);
+  const bool away = (mode == PRO_QUANT_AWAY || mode == PRO_NORM_AWAY);
   const int nb = dim / QK_K;
-  // x (or g), and gamma (or u); blocks past nb re-read the last, and values
-  // at or past n_valid (a multiple of 4, checked by the launch; they
-  // quantize as 0) read the last valid four, unused
+  // x and gamma; blocks past nb re-read the last, and values at or past
+  // n_valid (a multiple of 4, checked by the launch; they quantize as 0) read
+  // the last valid four, unused
   f32x4 xv[MAXB], wv[MAXB];
 #pragma unroll
   for (int j = 0; j < MAXB; ++j) {
     const int i = min(min(wave + 4 * j, nb - 1) * QK_K + 4 * lane, n_valid - 4);
     xv[j] = *reinterpret_cast<const f32x4*>(xt + i);
     if (norm) wv[j] = *reinterpret_cast<const f32x4*>(gamma + i);
-    if (swiglu) wv[j] = *reinterpret_cast<const f32x4*>(ut + i);
   }
   float rms = 1.0f;
   if (norm) {
@@ -184,19 +167,8 @@ __global__ void __launch_bounds__(256) k_quant_batch_r(const float* __restrict__
     const float w4[4] = {wv[j].x, wv[j].y, wv[j].z, wv[j].w};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      if (swiglu) {
-        const int i = b * QK_K + 4 * lane + k;
-        float h = 0.0f;
-        if (i < n_valid) {
-          const float g = v[k];
-          const float silu = g / (1.0f + exp_f32(-g));
-          h = silu * w4[k];
-        }
-        v[k] = h;
-      } else {
-        if (norm) v[k] = (v[k] * rms) * w4[k];
-        if (b * QK_K + 4 * lane + k >= n_valid) v[k] = 0.0f;
-      }
+      if (norm) v[k] = (v[k] * rms) * w4[k];
+      if (b * QK_K + 4 * lane + k >= n_valid) v[k] = 0.0f;
     }
     uint32_t packed;
     float d;
@@ -701,28 +673,17 @@ hipError_t launch_embed_batch(const WView& w, const int* tokens, int n_tok, int 
   return hipGetLastError();
 }
 
-hipError_t launch_quant_batch(const float* x, const float* u, int ld_x, const float* gamma, float eps, int dim,
-                              int n_valid, int mode, int n_tok, QuantBatch q, hipStream_t s) {
+hipError_t launch_quant_batch(const float* x, int ld_x, const float* gamma, float eps, int dim, int n_valid, int mode,
+                              int n_tok, QuantBatch q, hipStream_t s) {
   if (dim % QK_K) return hipErrorInvalidValue;
   // rows of up to 24 blocks load everything up front (k_quant_batch_r)
   const int nb = dim / QK_K;
   if (n_valid < 1 || n_valid > dim || n_valid > ld_x) return hipErrorInvalidValue;
   const bool up_front = ld_x % 4 == 0 && n_valid % 4 == 0;
-  if (up_front && nb <= 12)
-    hipLaunchKernelGGL(k_quant_batch_r<3>, quant_grid(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid,
-                       mode, n_tok, q.xh, q.xd, q.xbs);
-  else if (up_front && nb <= 24)
-    hipLaunchKernelGGL(k_quant_batch_r<6>, quant_grid(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid,
-                       mode, n_tok, q.xh, q.xd, q.xbs);
-  else
-    hipLaunchKernelGGL(k_quant_batch, quant_grid(n_tok), dim3(256), 0, s, x, u, ld_x, gamma, eps, dim, n_valid,
-                       mode, n_tok, q.xh, q.xd, q.xbs);
+  auto kern = up_front && nb <= 12 ? k_quant_batch_r<3> : up_front && nb <= 24 ? k_quant_batch_r<6> : k_quant_batch;
+  hipLaunchKernelGGL(kern, quant_grid(n_tok), dim3(256), 0, s, x, ld_x, gamma, eps, dim, n_valid, mode, n_tok, q.xh,
+                     q.xd, q.xbs);
   return hipGetLastError();
-}
-
-hipError_t launch_quant_batch_swiglu(const float* g, const float* u, int ld, int n_valid, int dim, int n_tok,
-                                     QuantBatch q, hipStream_t s) {
-  return launch_quant_batch(g, u, ld, nullptr, 0.0f, dim, n_valid, QB_SWIGLU, n_tok, q, s);
 }
 
 hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const QuantBatch& q, float* out, int ld_out,

@@ -51,10 +51,11 @@ def test_prefill_kv_and_tokens_match_per_token(ctx, case):
 
 # Prompt lengths around the GEMM's 16-token tiles and their grouping (one to
 # four tiles per work group, a last group that is not full) at shapes whose rows
-# end inside a row tile or pair (ffn 1400, 520), and rows enough for row
-# tiles in pairs (2304 at 200 tokens and more).
+# end inside a row tile or pair (ffn 1400 and 520; 1401 and 7, whose activations
+# also start at 4-byte offsets), and rows enough for row tiles in pairs (2304 at
+# 200 tokens and more).
 TILE_CASES = [(2, 512, 8, 2, 64, 1400, 2000, mix, n) for mix in (0, 1) for n in (2, 16, 17, 18, 33, 34, 50, 65, 66, 82, 114)]
-TILE_CASES += [(2, 256, 4, 1, 64, 520, 300, 0, 37), (2, 2304, 32, 8, 64, 5760, 1000, 0, 241), (2, 2304, 32, 8, 64, 5760, 1000, 1, 337)]
+TILE_CASES += [(2, 256, 4, 1, 64, 520, 300, 0, 37), (2, 256, 4, 1, 64, 1401, 300, 0, 21), (2, 256, 4, 1, 64, 7, 300, 0, 19), (2, 2304, 32, 8, 64, 5760, 1000, 0, 241), (2, 2304, 32, 8, 64, 5760, 1000, 1, 337)]
 
 
 @pytest.mark.parametrize("case", TILE_CASES, ids=lambda c: f"d{c[1]}-hd{c[4]}-mix{c[7]}-p{c[8]}")
