@@ -328,6 +328,20 @@ def test_rope(ctx, orc, pos):
     assert_bits(ctx.download(vd, np.float32, 2048), want)
 
 
+# a head's pairs as a kernel argument: one, and the most it holds; from device memory: one more, and the most
+@pytest.mark.parametrize("heads,head_dim", [(3, 2), (5, 128), (3, 130), (2, 1024)])
+@pytest.mark.parametrize("pos", [0, 1, 4095])
+def test_rope_head_dims(ctx, orc, heads, head_dim, pos):
+    rng = np.random.default_rng(pos + head_dim)
+    v = rand_act(rng, heads * head_dim)
+    announce(f"rope {heads}x{head_dim} pos={pos}")
+    vd = up(ctx, v)
+    mcpm.check(ctx.lib.mcpm_apply_rope(ctx.h, vd.ptr, pos, heads, head_dim, 5e6))
+    want = v.copy()
+    orc.or_apply_rope(P(want), pos, heads, head_dim, 5e6)
+    assert_bits(ctx.download(vd, np.float32, v.size), want)
+
+
 # (position, KV capacity): the launch covers the splits of every chunk count
 # up to the capacity's, which is not monotonic (64 chunks take 64 splits, 66
 # take 33), so positions well below a capacity of 65-128 chunks are included
