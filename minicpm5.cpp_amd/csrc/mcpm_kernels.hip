@@ -367,9 +367,10 @@ __global__ void __launch_bounds__(256 * AQ_GROUPS) k_attention_q8k(const float* 
 //
 // The score chains and the weighted V chains run on v_mfma_f32_16x16x4_f32:
 // its result is the chain of four fmas over k in order, each rounded to
-// nearest even with denormals kept (20 million results over normal, widely
-// spread and denormal operands, none different), so a token's scores and o_c
-// have the bits of the decode attention's fma chains.  Positions past a
+// nearest even with denormals kept (6 million results over normal, widely
+// spread, underflowing, denormal and cancelling operands, none different:
+// tests/cpp/mfma_check.hip), so a token's scores and o_c have the bits of the
+// decode attention's fma chains.  Positions past a
 // token's context score -1e9 and weigh 0; a 0 leaves the V chain as it is if
 // that V is finite, so a chunk with an infinity or NaN in V takes the plain
 // chains instead.  Layouts: A lane l holds row l%16, k = l/16; B column l%16, k

@@ -3,12 +3,15 @@ per-token decode path: the KV cache rows of every layer must be bit-identical
 to those left by one forward per token, and the generated continuation the
 same.  The per-token path itself is checked against the oracle elsewhere;
 the greedy test below also checks prefill + decode against the oracle."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
 import mcpm
 import oracle as O
-from conftest import announce, assert_bits
+from conftest import ROOT, announce, assert_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -63,6 +66,16 @@ def test_prefill_token_tiles(ctx, case):
     test_prefill_kv_and_tokens_match_per_token(ctx, case)
 
 
+# Row tiles in pairs at one, two and three token tiles, which take 8192 rows: o and
+# down (Q4_K, Q6_K; rows of 32 blocks, past the quantization's 24) and q, k and v
+WIDE_CASES = [(2, 8192, 4, 1, 64, 256, 300, 0, n) for n in (10, 26, 42)] + [(2, 256, 128, 16, 64, 256, 300, 0, n) for n in (10, 26)]
+
+
+@pytest.mark.parametrize("case", WIDE_CASES, ids=lambda c: f"d{c[1]}-h{c[2]}-p{c[8]}")
+def test_prefill_wide_matrices(ctx, case):
+    test_prefill_kv_and_tokens_match_per_token(ctx, case)
+
+
 # head_dim 128 and 96 (the attention's instances past 64), 32 (below), groups of 8, 3 and 1 query heads,
 # contexts that end inside a chunk, at its edge and one past it
 ATTN_CASES = [(2, 512, 16, 2, 128, 512, 300, 0, 70), (2, 512, 8, 4, 96, 512, 300, 0, 66), (2, 512, 8, 1, 32, 512, 300, 0, 65),
@@ -74,6 +87,16 @@ ATTN_CASES += [(2, 512, 20, 4, 64, 512, 300, 0, 90), (2, 512, 24, 4, 64, 512, 30
 @pytest.mark.parametrize("case", ATTN_CASES, ids=lambda c: f"h{c[2]}-kv{c[3]}-hd{c[4]}-p{c[8]}")
 def test_prefill_attention_shapes(ctx, case):
     test_prefill_kv_and_tokens_match_per_token(ctx, case)
+
+
+# normal, widely spread, softmax terms down to denormals, products that underflow, denormal values, sums that cancel
+@pytest.mark.parametrize("distribution", range(6))
+def test_fp32_mfma_is_the_fma_chain(distribution):
+    announce(f"fp32 mfma distribution {distribution}")
+    r = subprocess.run([os.path.join(ROOT, "tests", "cpp", "mfma_check"), str(distribution)], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert ", 0 differ" in r.stdout
 
 
 def test_prefill_infinite_v_leaves_earlier_tokens(ctx):
