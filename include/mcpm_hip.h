@@ -8,7 +8,10 @@
  *   2. Per-op entry points, one per kernel of the backend seam
  *      (src/ops/ops_internal.h:13-72) and of the ops API (include/ops.h:112-160).
  *      Activations are device pointers; calls are ordered on the context's
- *      stream and return after enqueueing.  mcpm_sync() waits for them.
+ *      stream and return after enqueueing, before their outputs are written:
+ *      mcpm_sync() waits for them.  mcpm_apply_rope, mcpm_execute_attention and
+ *      mcpm_execute_attention_noalloc wait for the stream themselves, so theirs
+ *      and every earlier call's outputs are complete on return.
  *   3. The engine: load_model / init_kv_cache / forward of MiniCPM5Engine
  *      (include/model.h:37-45) plus the decode loop of ChatSession
  *      (src/chat_session.cpp:154-186).

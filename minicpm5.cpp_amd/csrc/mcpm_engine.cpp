@@ -723,6 +723,7 @@ int prefill_pass(mcpm_engine* e, const int* tokens, int n, int pos0) {
   const mcpm_model_config& c = e->cfg;
   hipStream_t s = e->ctx->stream;
   PrefillBufs& b = e->pf;
+  const int n_cu = e->ctx->n_cu;
   const int qd = c.n_heads * c.head_dim, kvd = c.n_kv_heads * c.head_dim;
   const QuantBatch qb{b.xh, b.xd, b.xbs};
   MCPM_HIP(hipMemcpyAsync(b.tokens, tokens, n * sizeof(int), hipMemcpyHostToDevice, s));
@@ -745,19 +746,19 @@ int prefill_pass(mcpm_engine* e, const int* tokens, int n, int pos0) {
     float* vrows = vc + static_cast<size_t>(pos0) * kvd;
     const GemmMore v{view_of(L.wv), kvd, vrows, kvd};
     const bool with_v = v.w.type == MCPM_TYPE_Q6_K;
-    MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, s, &wk, kvd, krows, kvd, &rp, false,
+    MCPM_HIP(launch_gemm_q8k(wq, qd, nbd, n, qb, b.q, qd, false, n_cu, s, &wk, kvd, krows, kvd, &rp, false,
                              with_v ? &v : nullptr));
-    if (!with_v) MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, s));
+    if (!with_v) MCPM_HIP(launch_gemm_q8k(v.w, kvd, nbd, n, qb, vrows, kvd, false, n_cu, s));
     if (l == c.n_layers - 1) break;  // nothing after the last K/V rows reaches the cache
     MCPM_HIP(launch_attention_batch(b.q, kc, vc, c.n_heads, c.n_kv_heads, c.head_dim, e->max_chunks, part, tok_o,
                                     tok_mz, pos0, n, s));
     MCPM_HIP(launch_quant_batch_attn(part, tok_o, tok_mz, pos0, n, c.n_heads, c.head_dim, e->max_chunks, qb, s));
-    MCPM_HIP(launch_gemm_q8k(view_of(L.wo), c.dim, qd / QK_K, n, qb, b.x, c.dim, true, s));
+    MCPM_HIP(launch_gemm_q8k(view_of(L.wo), c.dim, qd / QK_K, n, qb, b.x, c.dim, true, n_cu, s));
     MCPM_HIP(launch_quant_batch(b.x, c.dim, L.ffn_norm, c.eps, c.dim, c.dim, PRO_NORM_AWAY, n, qb, s));
     // gate and up in one launch, h = silu(gate)*up written by its epilogue
-    MCPM_HIP(launch_gemm_q8k(wg, c.ffn, nbd, n, qb, b.g, c.ffn, false, s, &wu, c.ffn, nullptr, 0, nullptr, true));
+    MCPM_HIP(launch_gemm_q8k(wg, c.ffn, nbd, n, qb, b.g, c.ffn, false, n_cu, s, &wu, c.ffn, nullptr, 0, nullptr, true));
     MCPM_HIP(launch_quant_batch(b.g, c.ffn, nullptr, 0.0f, c.ffn_pad, c.ffn, PRO_QUANT_AWAY, n, qb, s));
-    MCPM_HIP(launch_gemm_q8k(view_of(L.wd), c.dim, c.ffn_pad / QK_K, n, qb, b.x, c.dim, true, s));
+    MCPM_HIP(launch_gemm_q8k(view_of(L.wd), c.dim, c.ffn_pad / QK_K, n, qb, b.x, c.dim, true, n_cu, s));
   }
   return MCPM_OK;
 }

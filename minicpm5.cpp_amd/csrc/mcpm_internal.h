@@ -374,7 +374,7 @@ struct GemmMore {
 // w2 / rows2 / out2 / ld_out2: a second matrix of w's type on the same
 // activations in the same launch.
 hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const QuantBatch& q, float* out, int ld_out,
-                           bool add, hipStream_t s, const WView* w2 = nullptr, int rows2 = 0, float* out2 = nullptr,
+                           bool add, int n_cu, hipStream_t s, const WView* w2 = nullptr, int rows2 = 0, float* out2 = nullptr,
                            int ld_out2 = 0, const GemmRope* rope = nullptr, bool swiglu = false,
                            const GemmMore* v = nullptr);
 hipError_t launch_attention_batch(const float* q, const float* kc, const float* vc, int n_heads, int n_kv_heads,

@@ -12,10 +12,6 @@
 //  * Sums of squares: 256 strided partials, then a pairwise tree.
 //  * Everything is compiled with -ffp-contract=off; fused multiply-adds are
 //    explicit.
-#include <algorithm>
-
-#include <cstdlib>
-
 #include "mcpm_attn.h"
 #include "mcpm_device.h"
 
@@ -377,10 +373,11 @@ __global__ void __launch_bounds__(256 * AQ_GROUPS) k_attention_q8k(const float* 
 // = l/16; D register i row 4*(l/16) + i, column l%16.  K, V and the softmax
 // terms are stored so that the 64 lanes of an operand read hit 64 banks.
 //
-// Bound by the MFMAs (32 cycles each, 128 per 16 rows and chunk at head_dim
-// 64: 29 us of MFMA time per launch for 1023 tokens, 32 heads); the
-// fma chains it replaces, one lane per (head, position) and (head, dim), took
-// 131 us per launch there, 89 now; 16 heads of 128 over 332 tokens 51.7 -> 24.6).
+// Of 90 us per launch for 1023 tokens and 32 heads of 64, a SIMD spends 28 in
+// MFMAs (32 cycles each, 128 per 16 rows and chunk) and 39 issuing the other
+// vector instructions (softmax, addresses); the rest is waiting, for what is not
+// measured.  The fma chains it replaces, one lane per (head, position) and (head,
+// dim): 131 us; 16 heads of 128 over 332 tokens 51.7 -> 24.6.
 template <int HDM, bool FULL>
 __global__ void __launch_bounds__(256) k_attention_tile(const float* __restrict__ q, const float* __restrict__ kc,
                                                         const float* __restrict__ vc, int n_heads, int n_kv_heads,

@@ -11,10 +11,11 @@
 //    group), then acc[m] = fma(d_x*d_w, float(isum[m]), acc[m]) over blocks in
 //    order, Q4_K's min chain, and ((a0+a4)+(a2+a6))+((a1+a5)+(a3+a7));
 //  * isum[m] for 16 rows x 16 tokens is one v_mfma_f32_16x16x32_f16: K runs
-//    over lane m's 32 bytes (8 sub-blocks x 4) with A = sub-block scale x
-//    weight code (over 64) and activation code (times 64).  Every product is an integer of at
-//    most 2048 in magnitude (exact in fp16) and every sum stays below 2^24
-//    (exact in fp32), so the MFMA result is isum[m] itself.  Q4_K: sc*q <= 945.
+//    over lane m's 32 bytes (8 sub-blocks x 4), activation code times 64 (the
+//    MFMA's A) against sub-block scale x weight code over 64 (its B).  Every
+//    product is an integer of at most 1920 * 127 in magnitude, its factors
+//    exact in fp16, and every sum stays below 2^24 (exact in fp32), so the MFMA
+//    result is isum[m] itself.  Q4_K: sc*q <= 945.
 //    Q6_K: the reference sums sc*q*x over lane m's bytes (q in 0..63) and
 //    subtracts 32*(sc[2m]*bsums[2m] + sc[2m+1]*bsums[2m+1]) -- sub-block m's
 //    offset, added into lane m -- then converts the int32 sum to float.
@@ -27,11 +28,9 @@
 //    integer does.
 //  * Q4_K's min sum (sum over sub-blocks of mn * pair-sum of bsums) is one
 //    more MFMA: mn[k/2] for k < 16 against bsums[k].
-// Attention per token is the decode kernel at that token's position.
+// The attention (k_attention_tile, mcpm_kernels.hip) forms the decode attention's
+// chains for tiles of tokens, and its partials are combined per token.
 #include <algorithm>
-#include <cstdio>
-#include <cstdlib>
-#include <type_traits>
 
 #include "mcpm_device.h"
 
@@ -248,17 +247,22 @@ __device__ __forceinline__ h2 splat2(float v) {
 // the row whose scales a lane decodes is the row of its results.  With K index
 // k = 4*s + i over sub-blocks s and bytes i, a lane's K range is sub-blocks 2g
 // and 2g+1: elements 64g + 4m + i and 64g + 32 + 4m + i for lane group m.
-// What bounds it: one wave per lane-group pair (not per row tile) lets a weight
-// operand, whose build costs more than its MFMA, serve up to four token tiles
-// in the registers that two took (a wave's chains are 8 floats per result where
-// all lane groups in one wave need 32), and a short prompt's rows run on four
-// waves at once.  Against a work group of four row tiles x all lane groups with
-// activations staged in LDS (a barrier per block): 1023 tokens of the 2.4B
-// shape, gate/up 198 -> 131 us, down 171 -> 125, the prompt 23.8 -> 20.5 ms;
-// 44 tokens, down 30 -> 19 us, v 12.5 -> 9.2, the prompt 5.2 -> 4.0 ms.  Past
-// 64 tokens the activation operands' reads (16 TB/s from the L2s for gate/up)
-// bound it, for short prompts each wave's own chain of blocks (0.3 us a block
-// of Q6_K, 0.2 of Q4_K) and the first weights from HBM.
+// One wave per lane-group pair (not per row tile) lets a weight operand, whose
+// build costs more than its MFMA, serve up to four token tiles in the registers
+// that two took (a wave's chains are 8 floats per result where all lane groups
+// in one wave need 32), and a short prompt's rows run on four waves at once.
+// Against a work group of four row tiles x all lane groups with activations
+// staged in LDS (a barrier per block): 1023 tokens of the 2.4B shape, gate/up 198
+// -> 131 us, down 171 -> 125, the prompt 23.8 -> 20.5 ms; 44 tokens, down 30 -> 19
+// us, the prompt 5.2 -> 4.0 ms.
+// What bounds it: past 64 tokens no unit alone (gate/up at 1023 tokens, by
+// counters: 17 TB/s of reads from the L2s, 96 % of them hits, vector instructions
+// issuing 60 % of the time, matrix cores busy 17 %), though half the reads, by a
+// second row tile per wave, took it from 204 us to 132.  For short prompts each wave's own chain of blocks: a launch on
+// weights from HBM takes about 5 us and, per block, 0.42 us for Q6_K and 0.31 for
+// Q4_K with one token tile, 0.12 more for each further one (2304 rows, down's 23
+// blocks at 11, 27, 44 and 59 tokens 14.8, 17.0, 20.1 and 23.0 us, o's 8 blocks
+// 7.5, 8.2, 9.3 and 10.6).
 // PF: blocks in flight (loads return in order, so weights and activations are
 // loaded equally far ahead).
 // bid: the work group's index in the GEMM's grid; s_acc: 8*NT*64 entries,
@@ -687,7 +691,7 @@ hipError_t launch_quant_batch(const float* x, int ld_x, const float* gamma, floa
 }
 
 hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const QuantBatch& q, float* out, int ld_out,
-                           bool add, hipStream_t s, const WView* w2, int rows2, float* out2, int ld_out2,
+                           bool add, int n_cu, hipStream_t s, const WView* w2, int rows2, float* out2, int ld_out2,
                            const GemmRope* rope, bool swiglu, const GemmMore* v) {
   if (w.type != MCPM_TYPE_Q4_K && w.type != MCPM_TYPE_Q6_K) return hipErrorInvalidValue;
   if (rows < 1 || nb < 1 || n_tok < 1) return hipErrorInvalidValue;
@@ -719,7 +723,7 @@ hipError_t launch_gemm_q8k(const WView& w, int rows, int nb, int n_tok, const Qu
     if ((tiles + n - 1) / n * (2 + n) < (tiles + NT - 1) / NT * (2 + NT)) NT = n;
   const int n_tg = (tiles + NT - 1) / NT;
   auto groups = [&](int rpg) { return (rows + rpg - 1) / rpg + (swiglu ? 0 : (std::max(rows2, 0) + rpg - 1) / rpg); };
-  const int RT = swiglu || (groups(32) + (av.rows + 31) / 32) * n_tg >= 256 ? 2 : 1;
+  const int RT = swiglu || (groups(32) + (av.rows + 31) / 32) * n_tg >= n_cu ? 2 : 1;
   auto blocks = [&](int n_rg) { return 8u * static_cast<unsigned>((n_rg / 8) * n_tg + ((n_rg % 8) * n_tg + 7) / 8); };
   const unsigned grid_a = blocks(groups(swiglu ? 16 : 16 * RT));
   const dim3 grid(grid_a + (pair ? blocks((av.rows + 16 * RT - 1) / (16 * RT)) : 0u));
