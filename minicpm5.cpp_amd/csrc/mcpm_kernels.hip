@@ -841,12 +841,13 @@ __global__ void __launch_bounds__(256) k_gemv_q8_0_rows(const WView w, const flo
 // wave for every SIMD (64 rows each; 65,536 rows on 256 CUs): 130560 x 1536 31.2
 // us, with 8 rows a work group 64.4, with 32 50.7; 65536 x 2304 35.7, 54.5, 44.7
 // (weights in the Infinity Cache; from HBM 50.0, 55.3, 45.8).  32 rows a work
-// group where that is one for every CU: 32768 x 2304 21.9 us, with 8 rows 27.1,
-// a lane per row 33.9; 12000 x 1024 6.1, 6.5, 10.8; 8192 x 2304 9.7, 9.2, 21.8.
+// group where 8 would take more than 12 work groups per CU: 32768 x 2304 21.9
+// us, with 8 rows 27.1, a lane per row 33.9; below that short rows lose by it
+// (18000 x 512 4.4 us, with 8 rows 3.7; 12000 x 1024 5.2, 4.5).
 hipError_t launch_gemv_q8_0(const WView& w, const float* x, float* out, int rows, int cols, int n_cu, hipStream_t s) {
   if (rows >= 256 * n_cu)
     hipLaunchKernelGGL(k_gemv_q8_0_rows, dim3((rows + 255) / 256), dim3(256), 0, s, w, x, out, rows, cols);
-  else if (rows > 32 * n_cu)
+  else if (rows > 96 * n_cu)
     hipLaunchKernelGGL(k_gemv_q8_0<32>, dim3((rows + 31) / 32), dim3(256), 0, s, w, x, out, rows, cols);
   else
     hipLaunchKernelGGL(k_gemv_q8_0<8>, dim3((rows + 7) / 8), dim3(256), 0, s, w, x, out, rows, cols);

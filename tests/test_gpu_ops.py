@@ -303,9 +303,9 @@ def test_gemv_f32_steps(ctx, orc, rows, cols):
     test_gemv_f32_activations_bit_exact(ctx, orc, mcpm.TYPE_F32, rows, cols, 1)
 
 
-# Q8_0 rows around the kernel's splits on 256 CUs: 8 rows a work group up to 8192 rows, 32 past that (its
+# Q8_0 rows around the kernel's splits on 256 CUs: 8 rows a work group up to 24576 rows, 32 past that (its
 # 64-block chunks whole, one past them, and ragged last work groups), a lane per row from 65536 on
-@pytest.mark.parametrize("rows,cols", [(8192, 32), (8193, 96), (8193, 64 * 32), (8200, 65 * 32), (65535, 32), (65536, 64), (70001, 96)])
+@pytest.mark.parametrize("rows,cols", [(24576, 32), (24577, 96), (24577, 64 * 32), (24580, 65 * 32), (65535, 32), (65536, 64), (70001, 96)])
 def test_gemv_q8_0_splits(ctx, orc, rows, cols):
     test_gemv_f32_activations_bit_exact(ctx, orc, mcpm.TYPE_Q8_0, rows, cols, 1)
 
